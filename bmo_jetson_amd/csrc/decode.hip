@@ -12,9 +12,8 @@
 //
 // Work decomposition (gfx950, wave64).  A workgroup of NW waves serves one
 // (batch entry, query head) unit; its waves take contiguous pieces of the
-// window.  Batches with many units use one wave per unit; small batches (B=1
-// decode) use 2 to 8 waves per unit (16 on request) so that enough waves run,
-// merging in LDS (a split across workgroups would have to merge through
+// window.  Batches with many units use one wave per unit, smaller ones 2 to
+// 8 (16 on request) so that enough waves run, merging in LDS (a split across workgroups would have to merge through
 // device-scope atomics, which serialize across the XCDs).  The ring stores
 // slots in groups of G = 64 / LPK keys
 // (ring_layout.hpp), LPK = head_dim / 32 blocks per key, so one group is one
@@ -313,6 +312,34 @@ __device__ __forceinline__ float half_of(uint32_t v) {
     return HI ? (float) h.y : (float) h.x;
 }
 
+// First group of wave w's run of n_grp groups split over NW waves (w <= NW).
+// Fused, wave 0 also quantizes and attends to the current token, which takes
+// it as long as about kNewGroups groups: of two or four waves its run is
+// shorter by that many (taking the new token alone it would leave 1 of 2 and
+// 3 of 4 waves for the window: at 384 units of 32 groups, RoPE, 17.5 us a
+// launch with two waves and 10.8 with four, against 13.8 and 10.0); of eight
+// or more, whose runs are that short, it takes the new token alone.
+constexpr int kNewGroups = 3;
+template <int NW, bool FUSED>
+__host__ __device__ constexpr int run_start(int w, int n_grp) {
+    if constexpr (!FUSED || NW == 1) return w * n_grp / NW;
+    const int left = n_grp - (NW - 1) * kNewGroups;
+    const int n0 = NW < 8 && left > 0 ? left / NW : 0;
+    return w == 0 ? 0 : n0 + (w - 1) * (n_grp - n0) / (NW > 1 ? NW - 1 : 1);
+}
+template <int NW, bool FUSED>
+constexpr bool runs_cover() {
+    for (int n = 1; n <= 200; ++n) {
+        if (run_start<NW, FUSED>(0, n) != 0 || run_start<NW, FUSED>(NW, n) != n) return false;
+        for (int w = 0; w < NW; ++w)
+            if (run_start<NW, FUSED>(w + 1, n) < run_start<NW, FUSED>(w, n)) return false;
+    }
+    return true;
+}
+static_assert(runs_cover<1, true>() && runs_cover<2, true>() && runs_cover<4, true>() && runs_cover<8, true>() &&
+                  runs_cover<16, true>() && runs_cover<8, false>(),
+              "every group belongs to one wave");
+
 }  // namespace
 
 template <int D, int NW, int PF, bool FUSED>
@@ -346,13 +373,7 @@ __global__ __launch_bounds__(64 * NW) void decode_kernel(DecodeParams p) {
     uint8_t *stripe = p.base + g.stripe_offset(p.layer, sid, kvh);
     float *out_row = p.out + (int64_t) unit * D;
 
-    // Contiguous group run of this wave.  Fused with several waves per
-    // unit, wave 0 quantizes and attends to the current token and the other
-    // waves split the window, so the new token's work is off the window's
-    // critical path.
-    constexpr bool kSplitNew = FUSED && NW > 1;
-    constexpr int NWW = kSplitNew ? NW - 1 : NW;  // waves that stream the window
-    const int ww = kSplitNew ? wave - 1 : wave;
+    // Contiguous group run of this wave: [run(wave), run(wave + 1)).
     int g0 = 0, n_it = 0;
 
     struct Grp {
@@ -414,8 +435,8 @@ __global__ __launch_bounds__(64 * NW) void decode_kernel(DecodeParams p) {
     const int window = (int) min((int64_t) pos + 1, (int64_t) g.n_ctx);
     const int cur = pos - (int) p.div_ctx.div((uint32_t) pos) * g.n_ctx;  // pos % n_ctx
     const int n_grp = (window + G - 1) / G;
-    g0 = ww < 0 ? 0 : ww * n_grp / NWW;
-    n_it = ww < 0 ? 0 : (ww + 1) * n_grp / NWW - g0;
+    g0 = run_start<NW, FUSED>(wave, n_grp);
+    n_it = run_start<NW, FUSED>(wave + 1, n_grp) - g0;
     if constexpr (NW > 1) {
 #pragma unroll
         for (int j = 0; j < NB - 1; ++j) load_clamped(j, buf[j]);
@@ -551,6 +572,21 @@ __global__ __launch_bounds__(64 * NW) void decode_kernel(DecodeParams p) {
         csum += w;
         block_axpy(T.v, w, acc);
     };
+    // acc sums w * c with codes 0..15 and the -8 w of every key is owed until
+    // the end (csum): over a long run that debt grows past the sums it is
+    // taken from, and their rounding with it.  It is paid every kSettle
+    // passes: 32 adds (error against 64 bits, one wave: 32 groups 6.3e-7
+    // without, 4.9e-7 with; 188 groups 1.3e-6 and 5.5e-7).  Eight waves'
+    // runs are short.
+    constexpr int kSettle = 16 / NB;
+    auto settle = [&]() {
+        const float c = (-8.0f / 16777216.0f) * csum;
+        const float c_hi = 16.0f * c;
+#pragma unroll
+        for (int e = 0; e < 32; ++e) acc[e] += e < 16 ? c : c_hi;
+        csum = 0.0f;
+    };
+    int settle_in = kSettle;
     // Steady state: every load is unconditional, so the wait before a group's
     // compute is for that group's loads only (a conditional prefetch would
     // make the compiler wait for the prefetch as well).  buf[u] holds group
@@ -561,6 +597,12 @@ __global__ __launch_bounds__(64 * NW) void decode_kernel(DecodeParams p) {
         for (int u = 0; u < NB; ++u) {
             load(t + u + NB - 1, buf[(u + NB - 1) % NB]);
             compute(t + u, buf[u]);
+        }
+        if constexpr (NW < 8) {
+            if (--settle_in == 0) {
+                settle();
+                settle_in = kSettle;
+            }
         }
     }
     // Tail: at most 2 * NB - 2 groups, loads only while groups remain.
@@ -668,7 +710,7 @@ struct Shape {
 };
 
 // The shapes launch_shape instantiates.
-constexpr Shape kShapes[] = {{1, 1}, {1, 2}, {1, 3}, {2, 1}, {4, 1}, {8, 1}, {8, 2}, {16, 1}};
+constexpr Shape kShapes[] = {{1, 1}, {1, 2}, {1, 3}, {2, 1}, {2, 2}, {4, 1}, {4, 2}, {8, 1}, {8, 2}, {16, 1}};
 
 constexpr bool shape_instantiated(Shape s) {
     for (const Shape &k : kShapes)
@@ -676,31 +718,46 @@ constexpr bool shape_instantiated(Shape s) {
     return false;
 }
 
-// Workgroup shape per call: one wave per (entry, head) unit with two groups
-// of loads in flight when there are enough units to fill the chip (measured
-// best over sustained runs of BASELINE config 3), else enough waves per unit
-// for about 512 waves in all.  Below 128 units, 8 waves per unit (B=1, 32
-// units, over a 32-layer model step whose windows come from HBM: 6.86 us
-// plain and 7.03 us fused per layer, against 7.44 and 8.16 us with 4 waves;
-// fused, wave 0 takes the new token), with two groups in flight per wave
-// when plain (5.62 against 5.74 us per layer with one) and one when fused
-// (5.87 against 5.89 us with two).  A window of fewer groups than waves
-// halves the waves, with one group in flight below 8 waves.
+// Workgroup shape per call, from the units (entry, head) and the window's
+// groups.  With two groups in flight a wave takes about 142 VGPRs, three
+// waves fit a SIMD and 3072 the chip; a unit gets as many waves (4, 2 or 1)
+// as leave every unit resident.  us per launch, 32 heads x d128, 512 slots
+// (32 groups) unless noted, 4 / 2 / 1 waves (RoPE + append; plain in
+// brackets):
+//   256 units   7.6 /  9.7 / 13.6 (6.6 / 8.7 / 12.3)
+//   768 units  13.5 / 13.9 / 15.3
+//   1024       18.3 / 15.8 / 16.7 (16.2 / 15.4 / 14.8)
+//   1536       23.7 / 22.7 / 24.2
+//   2048       29.8 / 31.3 / 28.6 (27.1 / 29.9 / 25.9)
+//   8192        108 /  106 /  105 (92.8 / 94.1 / 95.6)
+//   1024 units, 3000 slots  72.8 / 70.9 / 67.4 (71.1 / 68.9 / 64.5)
+// Past 2048 units, where one-wave units come in rounds, plain calls take
+// four waves again from 32 groups on (2560 units 32.6 against 34.3 us, 5120
+// 59.5 / 62.9, 3072 38.6 / 38.0; 8 groups, 8192 units: 40.3 / 28.9).  Between 768 and 1536 units two waves win by overlapping the prologues of
+// fused calls on short windows (up to 64 groups), and lose where the window's
+// bytes dominate.  Below 128 units 8 waves: one workgroup a CU at most, and
+// on long windows more waves still pay (3000 slots, 32 units 16.3 against
+// 17.5 us with 4, on 64 or more groups up to 256 units: 128 units 17.6 /
+// 19.0; 32 groups, 32 units, 7.4 / 7.1).  These units' calls are those of a
+// model's layer loop, whose results the next layer quantizes again: their
+// split of the window, and with it every rounding, is the same for all of
+// them.  Fewer groups than waves: fewer waves, but fused one more than the
+// groups, for the new token (depformer frame, one group: 200 / 207 us).
 constexpr Shape default_shape(int64_t units, int n_groups, bool fused) {
     Shape s{1, 2};
-    if (units < 128) s = Shape{8, fused ? 1 : 2};
-    else if (units < 256) s = Shape{4, 1};
-    else if (units < 512) s = Shape{2, 1};
-    while (s.nw > 1 && s.nw > n_groups) {  // no more waves than groups
-        s.nw /= 2;
-        s.pf = 1;
-    }
+    if (units < 128) s = Shape{8, fused && n_groups < 64 ? 1 : 2};
+    else if (units <= 256 && n_groups >= 64) s = Shape{8, 2};
+    else if (units <= 768) s = Shape{4, 2};
+    else if (units <= 1536 && fused && n_groups <= 64) s = Shape{2, 2};
+    else if (units > 2048 && !fused && n_groups >= 32) s = Shape{4, 2};
+    while (s.nw > 1 && s.nw > n_groups + (fused && n_groups == 1 ? 1 : 0)) s.nw /= 2;
+    if (n_groups == 1) s.pf = 1;
     return s;
 }
 
 constexpr bool default_shapes_instantiated() {
-    for (int64_t units : {1, 32, 127, 128, 255, 256, 511, 512, 1 << 20})
-        for (int n_groups = 1; n_groups <= 64; ++n_groups)
+    for (int64_t units : {1, 32, 127, 128, 256, 257, 768, 769, 1536, 1537, 2048, 2049, 1 << 20})
+        for (int n_groups = 1; n_groups <= 65; ++n_groups)
             for (bool fused : {false, true})
                 if (!shape_instantiated(default_shape(units, n_groups, fused))) return false;
     return true;
@@ -730,12 +787,14 @@ bool launch_shape(const DecodeParams &p, bool fused, hipStream_t stream, const S
     BMO_SHAPE(1, 2)
     BMO_SHAPE(1, 3)
     BMO_SHAPE(2, 1)
+    BMO_SHAPE(2, 2)
     BMO_SHAPE(4, 1)
+    BMO_SHAPE(4, 2)
     BMO_SHAPE(8, 1)
     BMO_SHAPE(8, 2)
     BMO_SHAPE(16, 1)
 #undef BMO_SHAPE
-    static_assert(sizeof(kShapes) / sizeof(kShapes[0]) == 8, "kShapes lists the shapes dispatched above");
+    static_assert(sizeof(kShapes) / sizeof(kShapes[0]) == 10, "kShapes lists the shapes dispatched above");
     return false;
 }
 

@@ -342,45 +342,50 @@ int bmo_kv_ring_append(bmo_kv_ring_t *r, int layer, int n_batch, const int *sess
     }
 }
 
-static int decode_common(bmo_kv_ring_t *r, const char *fn, bool fused, int layer, int n_batch,
-                         const int *session_ids, const int *pos, int n_heads, const float *q,
-                         const float *k_new, const float *v_new, float *out, float scale,
-                         float rope_theta, void *stream) {
+}  // extern "C"
+
+// The checks and the launch behind every ring decode call.
+int bmo::ring_decode_call(bmo_kv_ring_t *r, const char *fn, bool fused, const bmo::DecodeCall &c) {
     if (!r) return BMO_ATTN_ERR_NULL;
     try {
-        if (!pos || !q || !out || (fused && (!k_new || !v_new)))
+        if ((!c.pos && c.pos_host < 0) || !c.q || !c.out || (fused && (!c.k_new || !c.v_new)))
             return fail(r, BMO_ATTN_ERR_NULL, std::string(fn) + ": null pointer argument");
-        if (int rc = check_layer(r, layer, fn)) return rc;
-        if (n_batch <= 0 || n_batch > r->g.n_sessions)
+        if (int rc = check_layer(r, c.layer, fn)) return rc;
+        if (c.n_batch <= 0 || c.n_batch > r->g.n_sessions)
             return fail(r, BMO_ATTN_ERR_ARG, std::string(fn) + ": n_batch must be in [1, n_sessions]");
-        if (n_heads <= 0 || n_heads % r->g.n_kv_heads != 0)
+        if (c.n_heads <= 0 || c.n_heads % r->g.n_kv_heads != 0)
             return fail(r, BMO_ATTN_ERR_ARG,
                         std::string(fn) + ": n_heads must be a positive multiple of n_kv_heads");
-        if ((int64_t) n_batch * n_heads > INT_MAX)
+        if ((int64_t) c.n_batch * c.n_heads * c.n_layers > INT_MAX)
             return fail(r, BMO_ATTN_ERR_ARG, std::string(fn) + ": n_batch * n_heads exceeds INT_MAX");
-        if (!(scale > 0.0f)) scale = 1.0f / std::sqrt((float) r->g.head_dim);
+        const float scale = c.scale > 0.0f ? c.scale : 1.0f / std::sqrt((float) r->g.head_dim);
         if (!std::isfinite(scale))
             return fail(r, BMO_ATTN_ERR_ARG, std::string(fn) + ": scale must be finite");
-        if (rope_theta != 0.0f && !(rope_theta > 0.0f && std::isfinite(rope_theta)))
+        if (c.rope_theta != 0.0f && !(c.rope_theta > 0.0f && std::isfinite(c.rope_theta)))
             return fail(r, BMO_ATTN_ERR_ARG, std::string(fn) + ": rope_theta must be positive and finite");
         DeviceGuard dg(r->device);
         bmo::DecodeParams p{};
-        p.rope = rope_theta != 0.0f;
-        p.rope_r = p.rope ? std::pow((double) rope_theta, -2.0 / (double) r->g.head_dim) : 0.0;
+        p.rope = c.rope_theta != 0.0f;
+        p.rope_r = p.rope ? std::pow((double) c.rope_theta, -2.0 / (double) r->g.head_dim) : 0.0;
         p.base = r->mem;
         p.g = r->g;
-        p.layer = layer;
-        p.n_batch = n_batch;
-        p.n_heads = n_heads;
+        p.layer = c.layer;
+        p.n_layers = c.n_layers;
+        p.n_batch = c.n_batch;
+        p.n_heads = c.n_heads;
         p.n_kv = r->g.n_kv_heads;
-        p.session_ids = session_ids;
-        p.pos = pos;
-        p.q = q;
-        p.k_new = k_new;
-        p.v_new = v_new;
-        p.out = out;
+        p.session_ids = c.session_ids;
+        p.session0 = c.session0;
+        p.pos = c.pos;
+        p.pos_scalar = c.pos_host;
+        p.pos_out = c.pos_out;
+        p.pos_out_value = c.pos_out_value;
+        p.q = c.q;
+        p.k_new = c.k_new;
+        p.v_new = c.v_new;
+        p.out = c.out;
         p.qscale = scale * kLog2e;
-        if (!bmo::launch_decode(p, fused, (hipStream_t) stream))
+        if (!bmo::launch_decode(p, fused, (hipStream_t) c.stream))
             return fail(r, BMO_ATTN_ERR_ARG, std::string(fn) + ": unsupported head_dim");
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return hip_fail(r, e, fn);
@@ -390,6 +395,28 @@ static int decode_common(bmo_kv_ring_t *r, const char *fn, bool fused, int layer
         return fail(r, BMO_ATTN_ERR_INTERNAL, std::string(fn) + ": unknown exception");
     }
 }
+
+static int decode_common(bmo_kv_ring_t *r, const char *fn, bool fused, int layer, int n_batch,
+                         const int *session_ids, const int *pos, int n_heads, const float *q,
+                         const float *k_new, const float *v_new, float *out, float scale,
+                         float rope_theta, void *stream) {
+    bmo::DecodeCall c;
+    c.layer = layer;
+    c.n_batch = n_batch;
+    c.session_ids = session_ids;
+    c.pos = pos;
+    c.n_heads = n_heads;
+    c.q = q;
+    c.k_new = k_new;
+    c.v_new = v_new;
+    c.out = out;
+    c.scale = scale;
+    c.rope_theta = rope_theta;
+    c.stream = stream;
+    return bmo::ring_decode_call(r, fn, fused, c);
+}
+
+extern "C" {
 
 int bmo_kv_ring_decode(bmo_kv_ring_t *r, int layer, int n_batch, const int *session_ids,
                        const int *pos, int n_heads, const float *q, float *out, float scale,
@@ -767,6 +794,7 @@ void bmo_launch_decode_attention(const float *q_dev, const float *k_dev, const f
     }
     p.base = static_cast<uint8_t *>(k_cache_dev);
     p.layer = layer;
+    p.n_layers = 1;
     p.n_batch = 1;
     p.n_heads = n_heads;
     p.n_kv = n_kv_heads;

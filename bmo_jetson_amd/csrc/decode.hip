@@ -360,17 +360,19 @@ __global__ __launch_bounds__(64 * NW) void decode_kernel(DecodeParams p) {
     const int kk = lane / LPK;
     const int blk = lane % LPK;
 
-    const int unit = blockIdx.x;
-    const int b = (int) p.div_heads.div((uint32_t) unit);
-    const int h = unit - b * p.n_heads;
+    // blockIdx.x = entry * n_heads + head, blockIdx.y the layer of the launch
+    const int ll = blockIdx.y;
+    const int unit = ll * gridDim.x + blockIdx.x;
+    const int b = (int) p.div_heads.div(blockIdx.x);
+    const int h = blockIdx.x - b * p.n_heads;
 
     const RingGeom &g = p.g;
-    const int sid_in = p.session_ids ? p.session_ids[b] : b;
+    const int sid_in = p.session_ids ? p.session_ids[b] : p.session0 + b;
     const bool sid_ok = sid_in >= 0 && sid_in < g.n_sessions;
     const int sid = sid_ok ? sid_in : 0;  // an in-bounds stripe for loads issued before the check
     const int q_per_kv = p.q_per_kv;
     const int kvh = (int) p.div_qkv.div((uint32_t) h);
-    uint8_t *stripe = p.base + g.stripe_offset(p.layer, sid, kvh);
+    uint8_t *stripe = p.layer_base + ll * p.layer_bytes + ((int64_t) sid * g.n_kv_heads + kvh) * kGroupBytes;
     float *out_row = p.out + (int64_t) unit * D;
 
     // Contiguous group run of this wave: [run(wave), run(wave + 1)).
@@ -418,7 +420,7 @@ __global__ __launch_bounds__(64 * NW) void decode_kernel(DecodeParams p) {
     float xnew[NE];
     if constexpr (FUSED) {
         if (wave == 0) {
-            const float *src = (nb < LPK ? p.k_new : p.v_new) + ((int64_t) b * p.n_kv + kvh) * D +
+            const float *src = (nb < LPK ? p.k_new : p.v_new) + ((int64_t) (ll * p.n_batch + b) * p.n_kv + kvh) * D +
                                (nb % LPK) * kQK + gi * (NE / 2);
 #pragma unroll
             for (int t = 0; t < NE / 2; ++t) {
@@ -428,6 +430,7 @@ __global__ __launch_bounds__(64 * NW) void decode_kernel(DecodeParams p) {
         }
     }
     const int pos = p.pos ? p.pos[b] : p.pos_scalar;
+    if (p.pos_out && unit == 0 && threadIdx.x == 0) *p.pos_out = p.pos_out_value;
     if (!sid_ok || pos < 0) {
         for (int i = threadIdx.x; i < D; i += blockDim.x) out_row[i] = 0.0f;
         return;
@@ -698,7 +701,7 @@ namespace {
 
 template <int D, int NW, int PF>
 void launch_variant(const DecodeParams &p, bool fused, hipStream_t stream) {
-    const dim3 grid((unsigned) ((int64_t) p.n_batch * p.n_heads)), block(64 * NW);
+    const dim3 grid((unsigned) ((int64_t) p.n_batch * p.n_heads), (unsigned) p.n_layers), block(64 * NW);
     if (fused)
         hipLaunchKernelGGL((decode_kernel<D, NW, PF, true>), grid, block, 0, stream, p);
     else
@@ -801,11 +804,13 @@ bool launch_shape(const DecodeParams &p, bool fused, hipStream_t stream, const S
 }  // namespace
 
 bool launch_decode(const DecodeParams &params, bool fused, hipStream_t stream) {
-    const int64_t units = (int64_t) params.n_batch * params.n_heads;
+    const int64_t units = (int64_t) params.n_layers * params.n_batch * params.n_heads;
     if (units <= 0) return true;
     DecodeParams p = params;
     p.q_per_kv = p.n_heads / p.n_kv;
     p.div_heads = make_fastdiv((uint32_t) p.n_heads);
+    p.layer_base = p.base + p.g.stripe_offset(p.layer, 0, 0);
+    p.layer_bytes = p.g.n_groups * p.g.group_stride;
     p.div_qkv = make_fastdiv((uint32_t) p.q_per_kv);
     p.div_ctx = make_fastdiv((uint32_t) p.g.n_ctx);
     const Shape s = pick_shape(units, p.g.n_groups, fused);

@@ -7,6 +7,8 @@
 
 #include "ring_layout.hpp"
 
+struct bmo_kv_ring;
+
 namespace bmo {
 
 // Rows of fp32 K/V to quantize into ring slots.  Row r of the input goes to
@@ -50,23 +52,30 @@ inline FastDiv make_fastdiv(uint32_t d) {
 struct DecodeParams {
     uint8_t *base;  // ring allocation; the fused path writes the current slot
     RingGeom g;
-    int layer;
+    int layer;               // the first layer of the launch
+    int n_layers;            // layers of the launch: q, k_new, v_new and out hold one
+                             // [n_batch] row set per layer, all at the entries' positions
     int n_batch;
     int n_heads;
     int n_kv;                // logical kv heads: GQA map and k_new/v_new row stride
                              // (g.n_kv_heads is the allocated head count per stripe set)
-    const int *session_ids;  // device, nullable
+    const int *session_ids;  // device, or nullptr -> entry b is session session0 + b
+    int session0;
     const int *pos;          // device [n_batch], or nullptr -> pos_scalar
     int pos_scalar;
-    const float *q;      // [n_batch][n_heads][head_dim]
-    const float *k_new;  // [n_batch][n_kv][head_dim] (fused only)
+    int *pos_out;            // nullable: receives pos_out_value (a position the host knows;
+    int pos_out_value;       // no workgroup of the launch may read it)
+    const float *q;      // [n_layers][n_batch][n_heads][head_dim]
+    const float *k_new;  // [n_layers][n_batch][n_kv][head_dim] (fused only)
     const float *v_new;
-    float *out;          // [n_batch][n_heads][head_dim]
+    float *out;          // [n_layers][n_batch][n_heads][head_dim]
     float qscale;        // softmax scale * log2(e)
     int rope;            // nonzero: rotate q (and the fused k_new) by interleaved RoPE at pos
     double rope_r;       // theta^(-2/head_dim): pair i turns by pos * rope_r^i
-    // set by launch_decode: n_heads / n_kv and dividers by n_heads, by
-    // n_heads / n_kv and by g.n_ctx
+    // set by launch_decode: the first layer's group 0, the bytes of a layer,
+    // n_heads / n_kv and dividers by n_heads, by n_heads / n_kv and by g.n_ctx
+    uint8_t *layer_base;
+    int64_t layer_bytes;
     int q_per_kv;
     FastDiv div_heads, div_qkv, div_ctx;
 };
@@ -116,6 +125,29 @@ bool launch_gemv(const GemvParams &p, hipStream_t stream);
 // True when launch_prefill runs one attention kernel that quantizes and
 // commits the chunk itself (no staging stripes are read or written).
 bool prefill_is_direct(const PrefillParams &p);
+// One decode call on a ring (bmo_kv_ring_decode and the fused forms): the
+// entry points' arguments, and what only the session handle uses -- several
+// layers in one launch (buffers [n_layers][n_batch][...]), a session and a
+// position known to the host, and a device word that receives the position
+// after the call.
+struct DecodeCall {
+    int layer = 0;
+    int n_layers = 1;
+    int n_batch = 1;
+    const int *session_ids = nullptr;  // nullptr: entry b is session session0 + b
+    int session0 = 0;
+    const int *pos = nullptr;          // device; nullptr: every entry is at pos_host
+    int pos_host = -1;
+    int *pos_out = nullptr;
+    int pos_out_value = 0;
+    int n_heads = 0;
+    const float *q = nullptr, *k_new = nullptr, *v_new = nullptr;
+    float *out = nullptr;
+    float scale = 0.0f;
+    float rope_theta = 0.0f;
+    void *stream = nullptr;
+};
+int ring_decode_call(bmo_kv_ring *r, const char *fn, bool fused, const DecodeCall &c);
 // Message of the last ring call that failed on the calling thread (empty if
 // none): unlike the ring's own message, no other thread's call can replace it.
 const char *ring_thread_last_error();

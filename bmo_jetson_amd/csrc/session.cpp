@@ -44,6 +44,10 @@ struct bmo_attn_session {
     hipStream_t stream = nullptr;
     int *dev = nullptr;   // dev[0]: position read by every launch; dev[1]: the session id
     int64_t pos = 0;      // next position; dev[0] holds it once queued work has run
+    // what replay runs: a captured step (its buffers), or a recorded graph
+    bool step_set = false;
+    const float *step_q = nullptr, *step_k = nullptr, *step_v = nullptr;
+    float *step_out = nullptr;
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
     // what a replay of the graph does to the position: resets it to 0 first
@@ -116,15 +120,53 @@ int enqueue_advance(bmo_attn_session_t *s, const char *fn) {
     return BMO_ATTN_OK;
 }
 
-// Queues one token step on the handle's stream: every layer's fused append +
-// attention at the device position, then the position advances by one.
-int enqueue_step(bmo_attn_session_t *s, const float *q, const float *k, const float *v, float *out) {
+// Whether a step's output rows overlap its inputs: then a layer may read what
+// an earlier one wrote, and the layers run one after another.
+bool step_overlaps(const bmo_attn_session_t *s, const float *q, const float *k, const float *v, const float *out) {
+    const int64_t nq = (int64_t) s->n_layers * s->n_heads * s->head_dim;
+    const int64_t nk = (int64_t) s->n_layers * s->n_kv * s->head_dim;
+    auto meets = [&](const float *x, int64_t n) {
+        const uintptr_t a = (uintptr_t) x, b = (uintptr_t) out;
+        return a < b + 4 * (uintptr_t) nq && b < a + 4 * (uintptr_t) n;
+    };
+    return meets(q, nq) || meets(k, nk) || meets(v, nk);
+}
+
+// Queues one token step at position pos on the handle's stream: every
+// layer's fused append + attention, the last launch leaving pos + 1 as the
+// device position.  A step's inputs are all there when it begins, so one
+// launch serves every layer: at B = 1 a layer alone fills 32 of the chip's
+// 256 CUs and costs a launch, and the 32 of them took 230 us a step (512
+// slots, RoPE) and 579 us (3000 slots) one after another, against 26 and
+// 77 us in one launch.
+int enqueue_step(bmo_attn_session_t *s, int pos, const float *q, const float *k, const float *v, float *out) {
     const int64_t qs = (int64_t) s->n_heads * s->head_dim;
     const int64_t ks = (int64_t) s->n_kv * s->head_dim;
-    for (int l = 0; l < s->n_layers; ++l)
-        if (int rc = enqueue_layer(s, l, q + l * qs, k + l * ks, v + l * ks, out + l * qs, "token step"))
-            return rc;
-    return enqueue_advance(s, "token step");
+    const bool whole = s->n_layers <= 65535 && (int64_t) s->n_layers * s->n_heads <= INT_MAX &&
+                       !step_overlaps(s, q, k, v, out);
+    const int per = whole ? s->n_layers : 1;
+    for (int l = 0; l < s->n_layers; l += per) {
+        bmo::DecodeCall c;
+        c.layer = l;
+        c.n_layers = per;
+        c.session0 = s->session;
+        c.pos_host = pos;
+        if (l + per == s->n_layers) {
+            c.pos_out = s->dev;
+            c.pos_out_value = pos + 1;
+        }
+        c.n_heads = s->n_heads;
+        c.q = q + l * qs;
+        c.k_new = k + l * ks;
+        c.v_new = v + l * ks;
+        c.out = out + l * qs;
+        c.scale = s->scale;
+        c.rope_theta = s->rope_theta;
+        c.stream = s->stream;
+        if (int rc = bmo::ring_decode_call(s->ring, "token step", true, c))
+            return fail(s, rc, ring_message("token step"));
+    }
+    return BMO_ATTN_OK;
 }
 
 // Rejects a call that synchronizes or sets the position from the host while
@@ -298,11 +340,7 @@ int bmo_attn_session_forward(bmo_attn_session_t *s, int pos, const float *q, con
         if (!q || !k || !v || !out) return fail(s, BMO_ATTN_ERR_NULL, std::string(fn) + ": null pointer argument");
         if (int rc = check_pos(s, pos, fn)) return rc;
         DeviceGuard dg(s->device);
-        seek(s, pos);
-        if (int rc = enqueue_step(s, q, k, v, out)) {
-            (void) hipStreamSynchronize(s->stream);
-            // the device position is unknown after a partial step: set it again
-            bmo::launch_set_pos(s->dev, (int) s->pos, s->stream);
+        if (int rc = enqueue_step(s, pos, q, k, v, out)) {
             (void) hipStreamSynchronize(s->stream);
             return rc;
         }
@@ -321,20 +359,16 @@ int bmo_attn_session_capture(bmo_attn_session_t *s, const float *q, const float 
         if (int rc = check_not_capturing(s, fn)) return rc;
         if (!q || !k || !v || !out) return fail(s, BMO_ATTN_ERR_NULL, std::string(fn) + ": null pointer argument");
         DeviceGuard dg(s->device);
-        hipError_t e = hipStreamSynchronize(s->stream);
+        const hipError_t e = hipStreamSynchronize(s->stream);
         if (e != hipSuccess) return fail(s, BMO_ATTN_ERR_HIP, std::string(fn) + ": " + hipGetErrorString(e));
-        e = hipStreamBeginCapture(s->stream, hipStreamCaptureModeThreadLocal);
-        if (e != hipSuccess) return fail(s, BMO_ATTN_ERR_HIP, std::string(fn) + ": begin capture: " + hipGetErrorString(e));
-        const int rc = enqueue_step(s, q, k, v, out);
-        hipGraph_t graph = nullptr;
-        e = hipStreamEndCapture(s->stream, &graph);
-        if (rc != BMO_ATTN_OK) {
-            if (graph) (void) hipGraphDestroy(graph);
-            return rc;
-        }
-        if (e != hipSuccess || !graph)
-            return fail(s, BMO_ATTN_ERR_HIP, std::string(fn) + ": end capture: " + hipGetErrorString(e));
-        return keep_graph(s, graph, false, 1, fn);
+        drop_graph(s);
+        s->step_set = true;
+        s->step_q = q;
+        s->step_k = k;
+        s->step_v = v;
+        s->step_out = out;
+        s->last_error.clear();
+        return BMO_ATTN_OK;
     } catch (...) {
         return fail(s, BMO_ATTN_ERR_INTERNAL, std::string(fn) + ": unknown exception");
     }
@@ -343,7 +377,7 @@ int bmo_attn_session_capture(bmo_attn_session_t *s, const float *q, const float 
 int bmo_attn_session_has_graph(bmo_attn_session_t *s) {
     if (!s) return 0;
     std::lock_guard<std::mutex> lk(s->mu);
-    return s->exec ? 1 : 0;
+    return s->exec || s->step_set ? 1 : 0;
 }
 
 int bmo_attn_session_replay(bmo_attn_session_t *s, int pos) {
@@ -352,8 +386,14 @@ int bmo_attn_session_replay(bmo_attn_session_t *s, int pos) {
     const char *fn = "bmo_attn_session_replay";
     try {
         if (int rc = check_not_capturing(s, fn)) return rc;
-        if (!s->exec) return fail(s, BMO_ATTN_ERR_ARG, std::string(fn) + ": no captured step (call bmo_attn_session_capture first)");
+        if (!s->exec && !s->step_set)
+            return fail(s, BMO_ATTN_ERR_ARG, std::string(fn) + ": no captured step (call bmo_attn_session_capture first)");
         if (int rc = check_pos(s, pos, fn)) return rc;
+        if (s->step_set) {
+            DeviceGuard dg(s->device);
+            if (int rc = enqueue_step(s, pos, s->step_q, s->step_k, s->step_v, s->step_out)) return rc;
+            return finish(s, (int64_t) pos + 1, fn);
+        }
         if (!s->graph_resets && (int64_t) pos + s->graph_adv > INT_MAX)
             return fail(s, BMO_ATTN_ERR_ARG, std::string(fn) + ": the graph's steps would pass 2^31 - 1");
         DeviceGuard dg(s->device);

@@ -284,8 +284,8 @@ BMO_ATTN_API int bmo_positions_advance(int *pos_dev, int n, int delta, void *str
 /*
  * The attention part of the reference's bmo_handle (src/bmo_api.cpp:164-172):
  * one session of a ring, a HIP stream of its own (non-blocking, default
- * priority), a device-resident position that every launch reads (the
- * reference's pos_dev), and a mutex that serializes the handle's calls
+ * priority), a device-resident position (the reference's pos_dev), and a
+ * mutex that serializes the handle's calls
  * (src/bmo_api.cpp:28, :415).  A token step runs the fused append +
  * attention of every layer of the ring at one position (with RoPE when
  * rope_theta > 0) and advances the position, as bmo_forward_temporal2 does
@@ -326,17 +326,18 @@ BMO_ATTN_API void *bmo_attn_session_stream(bmo_attn_session_t *s);
 
 /* One token step at position pos (0 <= pos <= 2^31 - 2; any position, not
  * only the next one, as bmo_forward_temporal2 takes it,
- * src/bmo_api.cpp:365-511), launched eagerly on the handle's stream;
- * returns when out is written.  Afterwards the position is pos + 1. */
+ * src/bmo_api.cpp:365-511), launched eagerly on the handle's stream, all
+ * layers at once (one after another where out overlaps an input, so that a
+ * layer then sees what the layers before it wrote); returns when out is
+ * written.  Afterwards the position is pos + 1. */
 BMO_ATTN_API int bmo_attn_session_forward(bmo_attn_session_t *s, int pos, const float *q,
                                           const float *k, const float *v, float *out);
 
-/* Records one token step over these buffers into a HIP graph; the graph
- * reads the position from device memory and ends by advancing it.  Nothing
- * runs and the position does not change.  The buffers must stay valid while
- * the graph is kept.  A previous graph is replaced only once the new one is
- * instantiated (a failed capture keeps it).  Stands in for
- * bmo_capture_graphs (src/bmo_api.cpp:334-351). */
+/* Keeps these buffers as the step that replay runs: one token step, at the
+ * position replay is given, all layers in one launch.  Nothing runs and the
+ * position does not change.  The buffers must stay valid while the step is
+ * kept.  A previous step or graph is replaced (a failed capture keeps it).
+ * Stands in for bmo_capture_graphs (src/bmo_api.cpp:334-351). */
 BMO_ATTN_API int bmo_attn_session_capture(bmo_attn_session_t *s, const float *q, const float *k,
                                           const float *v, float *out);
 
@@ -344,8 +345,9 @@ BMO_ATTN_API int bmo_attn_session_capture(bmo_attn_session_t *s, const float *q,
  * src/bmo_api.cpp:353-359). */
 BMO_ATTN_API int bmo_attn_session_has_graph(bmo_attn_session_t *s);
 
-/* Replays the captured graph (bmo_attn_session_capture, or _capture_begin /
- * _end) on the handle's stream and returns when it is done; the captured
+/* Runs the captured step (bmo_attn_session_capture) or replays the captured
+ * graph (_capture_begin / _end) on the handle's stream and returns when it
+ * is done; the captured
  * buffers hold the inputs on entry and the outputs on return.  A graph that
  * does not begin with a reset runs at position pos (same range as forward;
  * replaying at the handle's current position costs one graph launch, another

@@ -31,6 +31,9 @@ struct bmo_kv_ring {
     uint8_t *stage = nullptr;  // prefill staging, grown on demand (guarded by stage_mu)
     int64_t stage_bytes = 0;
     std::mutex stage_mu;
+    uint8_t *readout = nullptr;  // pinned block buffer of the readout calls, made by the first
+    uint8_t *readout_dev = nullptr;  // ... as the device sees it (both guarded by readout_mu)
+    std::mutex readout_mu;
     std::mutex mu;           // guards last_error
     std::string last_error;
 };
@@ -122,62 +125,55 @@ float f16_to_f32_host(uint16_t h) {
     return f;
 }
 
-// Copies the groups holding slots [t0, t0+n) of one stripe to host, packed
-// back to back; *first receives the first group's index.
-// (One 1-D copy per group rather than one strided hipMemcpy2D: under
-// rocprofv3's kernel trace, hipMemcpy2D device-to-host returned wrong bytes
-// for these strides on MI355X while 1-D copies of the same groups were
-// exact.  These are the host-side readout paths, not the hot path.)
-hipError_t fetch_groups(const bmo_kv_ring_t *r, const uint8_t *stripe, int t0, int n,
-                        std::vector<uint8_t> &buf, int *first) {
-    const int G = bmo::keys_per_group(r->g.head_dim);
-    const int g0 = t0 / G, g1 = (t0 + n - 1) / G;
-    *first = g0;
-    buf.resize((size_t) (g1 - g0 + 1) * bmo::kGroupBytes);
-    for (int g = g0; g <= g1; ++g) {
-        const hipError_t e = hipMemcpy(buf.data() + (size_t) (g - g0) * bmo::kGroupBytes,
-                                       stripe + (int64_t) g * r->g.group_stride, bmo::kGroupBytes,
-                                       hipMemcpyDeviceToHost);
-        if (e != hipSuccess) return e;
+// Pinned buffer of a readout: large enough for a 512-slot, 32-head layer's K
+// or V at once; longer readouts pass through it in turn.
+constexpr int64_t kReadoutBytes = int64_t(2) << 20;
+
+// Moves the blocks of slots [t0, t0 + n) of one session's K or V in one
+// layer through the ring's pinned buffer.  each(i, blocks, count) is called
+// for blocks [i, i + count) of the readout, with the buffer's host side: to
+// read them after they left the ring, or (to_ring) to fill it before they
+// enter.  False on a HIP error.  Synchronous; the device's earlier work is
+// waited for first, on every stream, and one readout runs at a time.
+template <class F>
+bool readout(bmo_kv_ring_t *r, int layer, int session, int which, int t0, int n, bool to_ring, F each) {
+    std::lock_guard<std::mutex> lk(r->readout_mu);
+    if (hipDeviceSynchronize() != hipSuccess) return false;
+    if (!r->readout) {
+        void *dev = nullptr;
+        if (hipHostMalloc((void **) &r->readout, (size_t) kReadoutBytes, hipHostMallocDefault) != hipSuccess) {
+            r->readout = nullptr;
+            return false;
+        }
+        if (hipHostGetDevicePointer(&dev, r->readout, 0) != hipSuccess) {
+            (void) hipHostFree(r->readout);
+            r->readout = nullptr;
+            return false;
+        }
+        r->readout_dev = static_cast<uint8_t *>(dev);
     }
-    return hipSuccess;
-}
-
-// Writes packed groups back to their places in a stripe.
-hipError_t store_groups(const bmo_kv_ring_t *r, uint8_t *stripe, const std::vector<uint8_t> &buf,
-                        int first) {
-    const size_t n = buf.size() / bmo::kGroupBytes;
-    for (size_t i = 0; i < n; ++i) {
-        const hipError_t e = hipMemcpy(stripe + (int64_t) (first + (int64_t) i) * r->g.group_stride,
-                                       buf.data() + i * bmo::kGroupBytes, bmo::kGroupBytes,
-                                       hipMemcpyHostToDevice);
-        if (e != hipSuccess) return e;
+    const int64_t total = (int64_t) n * r->g.n_kv_heads * (r->g.head_dim / bmo::kQK);
+    const int64_t most = kReadoutBytes / bmo::readout_buffer_bytes(1) * (bmo::readout_buffer_bytes(1) / 18);
+    bmo::ReadoutParams p{};
+    p.base = r->mem;
+    p.g = r->g;
+    p.layer = layer;
+    p.session = session;
+    p.which = which;
+    p.slot0 = t0;
+    p.blocks = r->readout_dev;
+    for (p.first = 0; p.first < total; p.first += p.n_blocks) {
+        p.n_blocks = std::min(most, total - p.first);
+        if (to_ring) {
+            each(p.first, r->readout, p.n_blocks);
+            bmo::launch_import(p, nullptr);
+        } else {
+            bmo::launch_export(p, nullptr);
+        }
+        if (hipGetLastError() != hipSuccess || hipStreamSynchronize(nullptr) != hipSuccess) return false;
+        if (!to_ring) each(p.first, r->readout, p.n_blocks);
     }
-    return hipSuccess;
-}
-
-// ggml block (scale bits, 16 code bytes) of K (which 0) or V (which 1) at
-// slot, block blk, from packed groups starting at group `first`.
-void read_block(const bmo::RingGeom &g, const std::vector<uint8_t> &buf, int first, int which,
-                int slot, int blk, uint16_t *d, uint8_t *qs) {
-    const bmo::RingGeom pg = bmo::packed_stripe_geom(g);
-    const int64_t base = (int64_t) first * bmo::kGroupBytes;
-    const uint8_t *codes = buf.data() + (which == 0 ? pg.kcode_offset(slot, blk)
-                                                     : pg.vcode_offset(slot, blk)) - base;
-    const uint8_t flip = which == 0 ? bmo::kKCodeZero : 0;
-    for (int j = 0; j < 16; ++j) qs[j] = codes[j] ^ flip;
-    std::memcpy(d, buf.data() + pg.scale_offset(slot, blk) - base + 2 * which, 2);
-}
-
-void write_block(const bmo::RingGeom &g, std::vector<uint8_t> &buf, int first, int which,
-                 int slot, int blk, uint16_t d, const uint8_t *qs) {
-    const bmo::RingGeom pg = bmo::packed_stripe_geom(g);
-    const int64_t base = (int64_t) first * bmo::kGroupBytes;
-    uint8_t *codes = buf.data() + (which == 0 ? pg.kcode_offset(slot, blk)
-                                               : pg.vcode_offset(slot, blk)) - base;
-    const uint8_t flip = which == 0 ? bmo::kKCodeZero : 0;
-    for (int j = 0; j < 16; ++j) codes[j] = qs[j] ^ flip;
-    std::memcpy(buf.data() + pg.scale_offset(slot, blk) - base + 2 * which, &d, 2);
+    return true;
 }
 
 }  // namespace
@@ -254,6 +250,7 @@ void bmo_kv_ring_free(bmo_kv_ring_t *ring) {
         DeviceGuard dg(ring->device);
         if (ring->mem) (void) hipFree(ring->mem);
         if (ring->stage) (void) hipFree(ring->stage);
+        if (ring->readout) (void) hipHostFree(ring->readout);
     } catch (...) {
     }
     delete ring;
@@ -623,29 +620,21 @@ int bmo_kv_ring_copy_k_f32(bmo_kv_ring_t *r, int layer, int session, int t_start
         const int64_t need = (int64_t) n_positions * g.n_kv_heads * g.head_dim;
         if (need > (int64_t) max_floats) return BMO_ATTN_READ_ERR_SMALL;
         DeviceGuard dg(r->device);
-        if (hipDeviceSynchronize() != hipSuccess) return BMO_ATTN_READ_ERR_NULL;
-        const int D = g.head_dim;
-        const int nblk = D / bmo::kQK;
-        std::vector<uint8_t> buf;
-        int first = 0;
-        for (int h = 0; h < g.n_kv_heads; ++h) {
-            if (fetch_groups(r, r->mem + g.stripe_offset(layer, session, h), t_start, n_positions,
-                             buf, &first) != hipSuccess)
-                return BMO_ATTN_READ_ERR_NULL;
-            for (int ti = 0; ti < n_positions; ++ti) {
-                float *o = out + ((int64_t) ti * g.n_kv_heads + h) * D;
-                for (int b = 0; b < nblk; ++b) {
-                    uint16_t d16;
-                    uint8_t qs[16];
-                    read_block(g, buf, first, 0, t_start + ti, b, &d16, qs);
-                    const float d = f16_to_f32_host(d16);
-                    for (int j = 0; j < 16; ++j) {
-                        o[b * 32 + j] = (float) ((int) (qs[j] & 0x0F) - 8) * d;
-                        o[b * 32 + j + 16] = (float) ((int) (qs[j] >> 4) - 8) * d;
-                    }
+        const bool ok = readout(r, layer, session, 0, t_start, n_positions, false,
+                                [&](int64_t first, const uint8_t *blocks, int64_t count) {
+            for (int64_t i = 0; i < count; ++i) {
+                const uint8_t *b = blocks + i * 18;
+                float *o = out + (first + i) * bmo::kQK;
+                uint16_t d16;
+                std::memcpy(&d16, b, 2);
+                const float d = f16_to_f32_host(d16);
+                for (int j = 0; j < 16; ++j) {
+                    o[j] = (float) ((int) (b[2 + j] & 0x0F) - 8) * d;
+                    o[j + 16] = (float) ((int) (b[2 + j] >> 4) - 8) * d;
                 }
             }
-        }
+        });
+        if (!ok) return BMO_ATTN_READ_ERR_NULL;
         return (int) need;
     } catch (...) {
         return BMO_ATTN_READ_ERR_NULL;
@@ -665,22 +654,11 @@ int64_t bmo_kv_ring_export_q4_0(bmo_kv_ring_t *r, int layer, int session, int wh
         const int64_t need = (int64_t) n_positions * g.n_kv_heads * nblk * 18;
         if (need > max_bytes) return BMO_ATTN_READ_ERR_SMALL;
         DeviceGuard dg(r->device);
-        if (hipDeviceSynchronize() != hipSuccess) return BMO_ATTN_READ_ERR_NULL;
-        uint8_t *dst = static_cast<uint8_t *>(out);
-        std::vector<uint8_t> buf;
-        int first = 0;
-        for (int h = 0; h < g.n_kv_heads; ++h) {
-            if (fetch_groups(r, r->mem + g.stripe_offset(layer, session, h), t_start, n_positions,
-                             buf, &first) != hipSuccess)
-                return BMO_ATTN_READ_ERR_NULL;
-            for (int ti = 0; ti < n_positions; ++ti)
-                for (int b = 0; b < nblk; ++b) {
-                    uint8_t *blkp = dst + (((int64_t) ti * g.n_kv_heads + h) * nblk + b) * 18;
-                    uint16_t d16;
-                    read_block(g, buf, first, which, t_start + ti, b, &d16, blkp + 2);
-                    std::memcpy(blkp, &d16, 2);
-                }
-        }
+        const bool ok = readout(r, layer, session, which, t_start, n_positions, false,
+                                [&](int64_t first, const uint8_t *blocks, int64_t count) {
+            std::memcpy(static_cast<uint8_t *>(out) + first * 18, blocks, (size_t) count * 18);
+        });
+        if (!ok) return BMO_ATTN_READ_ERR_NULL;
         return need;
     } catch (...) {
         return BMO_ATTN_READ_ERR_NULL;
@@ -700,25 +678,11 @@ int64_t bmo_kv_ring_import_q4_0(bmo_kv_ring_t *r, int layer, int session, int wh
         const int64_t need = (int64_t) n_positions * g.n_kv_heads * nblk * 18;
         if (n_bytes < need) return BMO_ATTN_READ_ERR_SMALL;
         DeviceGuard dg(r->device);
-        if (hipDeviceSynchronize() != hipSuccess) return BMO_ATTN_READ_ERR_NULL;
-        const uint8_t *src = static_cast<const uint8_t *>(in);
-        std::vector<uint8_t> buf;
-        int first = 0;
-        for (int h = 0; h < g.n_kv_heads; ++h) {
-            uint8_t *stripe = r->mem + g.stripe_offset(layer, session, h);
-            // read-modify-write: a group also holds other slots and the other
-            // half of each scale dword
-            if (fetch_groups(r, stripe, t_start, n_positions, buf, &first) != hipSuccess)
-                return BMO_ATTN_READ_ERR_NULL;
-            for (int ti = 0; ti < n_positions; ++ti)
-                for (int b = 0; b < nblk; ++b) {
-                    const uint8_t *blkp = src + (((int64_t) ti * g.n_kv_heads + h) * nblk + b) * 18;
-                    uint16_t d16;
-                    std::memcpy(&d16, blkp, 2);
-                    write_block(g, buf, first, which, t_start + ti, b, d16, blkp + 2);
-                }
-            if (store_groups(r, stripe, buf, first) != hipSuccess) return BMO_ATTN_READ_ERR_NULL;
-        }
+        const bool ok = readout(r, layer, session, which, t_start, n_positions, true,
+                                [&](int64_t first, uint8_t *blocks, int64_t count) {
+            std::memcpy(blocks, static_cast<const uint8_t *>(in) + first * 18, (size_t) count * 18);
+        });
+        if (!ok) return BMO_ATTN_READ_ERR_NULL;
         return need;
     } catch (...) {
         return BMO_ATTN_READ_ERR_NULL;

@@ -101,6 +101,21 @@ struct PrefillParams {
     int n_resident;  // set by launch_prefill: workgroups the device runs at once (0: unknown)
 };
 
+// n_blocks blocks, from block `first` on, of one session's K (which 0) or V
+// (which 1) slots slot0.. in one layer, [slots][n_kv_heads][head_dim / 32],
+// to or from ggml blocks (readout.hip).
+struct ReadoutParams {
+    uint8_t *base;  // ring allocation
+    RingGeom g;
+    int layer;
+    int session;
+    int which;
+    int slot0;
+    int64_t first;
+    int64_t n_blocks;
+    uint8_t *blocks;  // readout_buffer_bytes(n_blocks) bytes, 16-byte aligned
+};
+
 // Launchers enqueue only; they leave launch errors for the caller's
 // hipGetLastError().  launch_decode returns false for an unsupported head_dim.
 void launch_append(const AppendParams &p, hipStream_t stream);
@@ -110,6 +125,11 @@ bool launch_decode(const DecodeParams &p, bool fused, hipStream_t stream);
 // stage, attend, commit (three kernels in stream order); false for an
 // unsupported head_dim.
 bool launch_prefill(const PrefillParams &p, hipStream_t stream);
+
+// Bytes of the block buffer of n_blocks blocks: whole workgroups.
+int64_t readout_buffer_bytes(int64_t n_blocks);
+void launch_export(const ReadoutParams &p, hipStream_t stream);
+void launch_import(const ReadoutParams &p, hipStream_t stream);
 
 struct GemvParams {
     const uint8_t *w;  // ggml block_q4_0 rows [rows][cols/32] (18 bytes each)

@@ -92,15 +92,4 @@ __host__ __device__ inline RingGeom make_geom(int n_layers, int n_sessions, int 
     return g;
 }
 
-// A stripe's groups packed back to back (group_stride = kGroupBytes): the
-// layout of a host copy of one stripe's groups.
-__host__ __device__ inline RingGeom packed_stripe_geom(const RingGeom &g) {
-    RingGeom p = g;
-    p.n_layers = 1;
-    p.n_sessions = 1;
-    p.n_kv_heads = 1;
-    p.group_stride = kGroupBytes;
-    return p;
-}
-
 }  // namespace bmo

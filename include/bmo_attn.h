@@ -237,7 +237,10 @@ BMO_ATTN_API int bmo_kv_ring_prefill_noalloc(bmo_kv_ring_t *ring, int layer, int
                                              const uint16_t *k, const uint16_t *v,
                                              float *out, float scale, void *stream);
 
-/* ---- readout / export ------------------------------------------------------- */
+/* ---- readout / export -------------------------------------------------------
+ * These calls wait for the device's earlier work and run one at a time per
+ * ring; the first on a ring allocates 2 MiB of pinned host memory, kept until
+ * the ring is freed, which their blocks pass through. */
 
 /* Copies slots [t_start, t_start+n_positions) of layer's K for one session as
  * fp32 into HOST memory, layout (n_positions, n_kv_heads, head_dim); blocks

@@ -342,8 +342,12 @@ static_assert(runs_cover<1, true>() && runs_cover<2, true>() && runs_cover<4, tr
 
 }  // namespace
 
-template <int D, int NW, int PF, bool FUSED>
-__global__ __launch_bounds__(64 * NW) void decode_kernel(DecodeParams p) {
+// NW = R * S waves serve R query heads of one kv head, S waves each (R > 1:
+// grouped queries): the R heads' waves walk the same groups in step, so all
+// but the first find them in the CU's cache.
+template <int D, int S, int PF, bool FUSED, int R>
+__global__ __launch_bounds__(64 * R * S) void decode_kernel(DecodeParams p) {
+    constexpr int NW = R * S;
     constexpr int LPK = D / kQK;   // lanes (blocks) per key
     constexpr int G = 64 / LPK;    // keys per group = per wave iteration
     constexpr int NB = PF + 1;     // resident groups per wave
@@ -356,15 +360,22 @@ __global__ __launch_bounds__(64 * NW) void decode_kernel(DecodeParams p) {
     __shared__ float2 s_rope[NW][D / 2];
 
     const int lane = threadIdx.x & 63;
-    const int wave = threadIdx.x >> 6;
+    // Wave-uniform where that measured faster (frame 202 against 206 us, 64
+    // sessions 103.8 / 104.2); with several streaming waves and two groups in
+    // flight a branch on it costs a wait for every load (12 sessions, RoPE:
+    // 158 us against 150).
+    const int wave_v = (int) threadIdx.x >> 6;
+    const int wave = S == 1 || PF == 1 ? __builtin_amdgcn_readfirstlane(wave_v) : wave_v;
+    const int ws = wave % S;  // this wave's place among its head's S
     const int kk = lane / LPK;
     const int blk = lane % LPK;
 
-    // blockIdx.x = entry * n_heads + head, blockIdx.y the layer of the launch
+    // blockIdx.x = entry * (n_heads / R) + R query heads, blockIdx.y the
+    // layer of the launch
     const int ll = blockIdx.y;
-    const int unit = ll * gridDim.x + blockIdx.x;
     const int b = (int) p.div_heads.div(blockIdx.x);
-    const int h = blockIdx.x - b * p.n_heads;
+    const int h = ((int) blockIdx.x - b * p.heads_r) * R + wave / S;
+    const int64_t unit = ((int64_t) ll * p.n_batch + b) * p.n_heads + h;
 
     const RingGeom &g = p.g;
     const int sid_in = p.session_ids ? p.session_ids[b] : p.session0 + b;
@@ -373,9 +384,9 @@ __global__ __launch_bounds__(64 * NW) void decode_kernel(DecodeParams p) {
     const int q_per_kv = p.q_per_kv;
     const int kvh = (int) p.div_qkv.div((uint32_t) h);
     uint8_t *stripe = p.layer_base + ll * p.layer_bytes + ((int64_t) sid * g.n_kv_heads + kvh) * kGroupBytes;
-    float *out_row = p.out + (int64_t) unit * D;
+    float *out_row = p.out + unit * D;
 
-    // Contiguous group run of this wave: [run(wave), run(wave + 1)).
+    // Contiguous group run of this wave: [run(ws), run(ws + 1)).
     int g0 = 0, n_it = 0;
 
     struct Grp {
@@ -403,12 +414,12 @@ __global__ __launch_bounds__(64 * NW) void decode_kernel(DecodeParams p) {
     // the position is read (the scalar read's latency then overlaps its
     // own); with one wave per unit the run starts at group 0 whatever the
     // position, so the first groups go out ahead of it as well.
-    if constexpr (NW == 1) {
+    if constexpr (S == 1) {
 #pragma unroll
         for (int j = 0; j < NB - 1; ++j) load_clamped(j, buf[j]);
     }
-    prep_load<D>(p.q + (int64_t) unit * D, lane, q_lo, q_hi);
-    // Fused: wave 0 holds the current token's K and V rows spread over its
+    prep_load<D>(p.q + unit * D, lane, q_lo, q_hi);
+    // Fused: a head's wave 0 holds the current token's K and V rows spread over its
     // lanes for the lane-parallel quantizer, BL lanes per block: lane l
     // takes block nb = l / BL (K block nb for nb < LPK, else V block
     // nb - LPK), elements gi*NE/2 + t and gi*NE/2 + t + 16 of it (t < NE/2),
@@ -419,7 +430,7 @@ __global__ __launch_bounds__(64 * NW) void decode_kernel(DecodeParams p) {
     const int gi = lane % BL;
     float xnew[NE];
     if constexpr (FUSED) {
-        if (wave == 0) {
+        if (ws == 0) {
             const float *src = (nb < LPK ? p.k_new : p.v_new) + ((int64_t) (ll * p.n_batch + b) * p.n_kv + kvh) * D +
                                (nb % LPK) * kQK + gi * (NE / 2);
 #pragma unroll
@@ -432,15 +443,16 @@ __global__ __launch_bounds__(64 * NW) void decode_kernel(DecodeParams p) {
     const int pos = p.pos ? p.pos[b] : p.pos_scalar;
     if (p.pos_out && unit == 0 && threadIdx.x == 0) *p.pos_out = p.pos_out_value;
     if (!sid_ok || pos < 0) {
-        for (int i = threadIdx.x; i < D; i += blockDim.x) out_row[i] = 0.0f;
+        if (ws == 0)
+            for (int i = lane; i < D; i += 64) out_row[i] = 0.0f;
         return;
     }
     const int window = (int) min((int64_t) pos + 1, (int64_t) g.n_ctx);
     const int cur = pos - (int) p.div_ctx.div((uint32_t) pos) * g.n_ctx;  // pos % n_ctx
     const int n_grp = (window + G - 1) / G;
-    g0 = run_start<NW, FUSED>(wave, n_grp);
-    n_it = run_start<NW, FUSED>(wave + 1, n_grp) - g0;
-    if constexpr (NW > 1) {
+    g0 = run_start<S, FUSED>(ws, n_grp);
+    n_it = run_start<S, FUSED>(ws + 1, n_grp) - g0;
+    if constexpr (S > 1) {
 #pragma unroll
         for (int j = 0; j < NB - 1; ++j) load_clamped(j, buf[j]);
     }
@@ -472,7 +484,7 @@ __global__ __launch_bounds__(64 * NW) void decode_kernel(DecodeParams p) {
     for (int e = 0; e < 32; ++e) acc[e] = 0.0f;
 
     if constexpr (FUSED) {
-        if (wave == 0) {
+        if (ws == 0) {
             // The current token's blocks, quantized by the whole wave (BL
             // lanes per block); the K and V codes and scales of block blk
             // then move to lane blk (kk == 0), which attends to the new key.
@@ -480,7 +492,7 @@ __global__ __launch_bounds__(64 * NW) void decode_kernel(DecodeParams p) {
             constexpr int LPD = 4 / HE;  // lanes per code dword
             if (p.rope) {
                 // K pairs (2m, 2m+1) of the head turn by table entry m
-                const float2 *tab = s_rope[0] + (nb % LPK) * 16;
+                const float2 *tab = s_rope[wave] + (nb % LPK) * 16;
                 if constexpr (HE == 2) {
                     float a0 = xnew[0], b0 = xnew[1], a1 = xnew[2], b1 = xnew[3];
                     rope_pair(a0, b0, tab[gi]);
@@ -601,7 +613,7 @@ __global__ __launch_bounds__(64 * NW) void decode_kernel(DecodeParams p) {
             load(t + u + NB - 1, buf[(u + NB - 1) % NB]);
             compute(t + u, buf[u]);
         }
-        if constexpr (NW < 8) {
+        if constexpr (S < 8) {
             if (--settle_in == 0) {
                 settle();
                 settle_in = kSettle;
@@ -638,10 +650,10 @@ __global__ __launch_bounds__(64 * NW) void decode_kernel(DecodeParams p) {
     for (int i = 0; i < 16; ++i) {
         z[i] = swap_sum32(acc[2 * i], acc[2 * i + 1]);
     }
-    float ws[8];
+    float zs[8];
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
-        ws[j] = row_block_sum<LPK>(swap_sum16(z[2 * j], z[2 * j + 1]));
+        zs[j] = row_block_sum<LPK>(swap_sum16(z[2 * j], z[2 * j + 1]));
     }
     // Lane l (row r = l / 16) now holds elements blk * 32 + 4 j + mr, j < 8,
     // mr = {0, 2, 1, 3}[r], replicated over the REP = 16 / LPK lanes of its
@@ -657,19 +669,20 @@ __global__ __launch_bounds__(64 * NW) void decode_kernel(DecodeParams p) {
     float o[NJ];
 #pragma unroll
     for (int jj = 0; jj < NJ; ++jj) {
-        float v = ws[jj * REP];
+        float v = zs[jj * REP];
 #pragma unroll
-        for (int r = 1; r < REP; ++r) v = (ri == r) ? ws[jj * REP + r] : v;
+        for (int r = 1; r < REP; ++r) v = (ri == r) ? zs[jj * REP + r] : v;
         o[jj] = v;
     }
     const int obase = blk * kQK + 4 * ri + mr;  // element of o[jj] is obase + 4 REP jj
     float L = l_wave;  // 2^24 times the weight sum of the whole window
-    if constexpr (NW == 1) {
+    if constexpr (S == 1) {
         const float inv_l = (L > 0.0f) ? 16777216.0f / L : 0.0f;
 #pragma unroll
         for (int jj = 0; jj < NJ; ++jj) out_row[obase + 4 * REP * jj] = o[jj] * inv_l;
     } else {
-        // Merge the waves: each writes its row of sums and its (max, sum).
+        // Merge each head's waves: each writes its row of sums and its (max,
+        // sum); thread t then makes element t % D of head t / D.
 #pragma unroll
         for (int jj = 0; jj < NJ; ++jj) s_acc[wave * D + obase + 4 * REP * jj] = o[jj];
         if (lane == 0) {
@@ -677,47 +690,55 @@ __global__ __launch_bounds__(64 * NW) void decode_kernel(DecodeParams p) {
             s_l[wave] = l_wave;
         }
         __syncthreads();
-        float M = s_m[0];
+        static_assert(64 * NW >= R * D, "a thread per output");
+        const int rh = R == 1 ? 0 : (int) threadIdx.x / D;
+        const int el = (int) threadIdx.x - rh * D;
+        if (threadIdx.x < R * D) {
+            float M = s_m[rh * S];
 #pragma unroll
-        for (int w = 1; w < NW; ++w) M = fmaxf(M, s_m[w]);
-        float fw[NW];
-        L = 0.0f;
+            for (int w = 1; w < S; ++w) M = fmaxf(M, s_m[rh * S + w]);
+            float fw[S];
+            L = 0.0f;
 #pragma unroll
-        for (int w = 0; w < NW; ++w) {
-            fw[w] = __builtin_amdgcn_exp2f(s_m[w] - M);
-            L = __builtin_fmaf(fw[w], s_l[w], L);
-        }
-        const float inv_l = (L > 0.0f) ? 16777216.0f / L : 0.0f;
-        if (threadIdx.x < D) {
+            for (int w = 0; w < S; ++w) {
+                fw[w] = __builtin_amdgcn_exp2f(s_m[rh * S + w] - M);
+                L = __builtin_fmaf(fw[w], s_l[rh * S + w], L);
+            }
+            const float inv_l = (L > 0.0f) ? 16777216.0f / L : 0.0f;
             float a = 0.0f;
 #pragma unroll
-            for (int w = 0; w < NW; ++w) a = __builtin_fmaf(fw[w], s_acc[w * D + threadIdx.x], a);
-            out_row[threadIdx.x] = a * inv_l;
+            for (int w = 0; w < S; ++w) a = __builtin_fmaf(fw[w], s_acc[(rh * S + w) * D + el], a);
+            (out_row + (rh - wave / S) * D)[el] = a * inv_l;
         }
     }
 }
 
 namespace {
 
-template <int D, int NW, int PF>
-void launch_variant(const DecodeParams &p, bool fused, hipStream_t stream) {
-    const dim3 grid((unsigned) ((int64_t) p.n_batch * p.n_heads), (unsigned) p.n_layers), block(64 * NW);
+template <int D, int S, int PF, int R>
+void launch_variant(const DecodeParams &params, bool fused, hipStream_t stream) {
+    DecodeParams p = params;
+    p.heads_r = p.n_heads / R;
+    p.div_heads = make_fastdiv((uint32_t) p.heads_r);
+    const dim3 grid((unsigned) ((int64_t) p.n_batch * p.heads_r), (unsigned) p.n_layers), block(64 * R * S);
     if (fused)
-        hipLaunchKernelGGL((decode_kernel<D, NW, PF, true>), grid, block, 0, stream, p);
+        hipLaunchKernelGGL((decode_kernel<D, S, PF, true, R>), grid, block, 0, stream, p);
     else
-        hipLaunchKernelGGL((decode_kernel<D, NW, PF, false>), grid, block, 0, stream, p);
+        hipLaunchKernelGGL((decode_kernel<D, S, PF, false, R>), grid, block, 0, stream, p);
 }
 
+// Waves per unit, groups in flight per wave, query heads per workgroup.
 struct Shape {
-    int nw, pf;
+    int nw, pf, r;
 };
 
 // The shapes launch_shape instantiates.
-constexpr Shape kShapes[] = {{1, 1}, {1, 2}, {1, 3}, {2, 1}, {2, 2}, {4, 1}, {4, 2}, {8, 1}, {8, 2}, {16, 1}};
+constexpr Shape kShapes[] = {{1, 1, 1}, {1, 2, 1}, {2, 1, 1}, {2, 2, 1}, {4, 1, 1}, {4, 2, 1}, {8, 1, 1}, {8, 2, 1},
+                             {1, 2, 2}, {2, 2, 2}, {4, 2, 2}, {1, 2, 4}};
 
 constexpr bool shape_instantiated(Shape s) {
     for (const Shape &k : kShapes)
-        if (k.nw == s.nw && k.pf == s.pf) return true;
+        if (k.nw == s.nw && k.pf == s.pf && k.r == s.r) return true;
     return false;
 }
 
@@ -746,13 +767,26 @@ constexpr bool shape_instantiated(Shape s) {
 // split of the window, and with it every rounding, is the same for all of
 // them.  Fewer groups than waves: fewer waves, but fused one more than the
 // groups, for the new token (depformer frame, one group: 200 / 207 us).
-constexpr Shape default_shape(int64_t units, int n_groups, bool fused) {
-    Shape s{1, 2};
-    if (units < 128) s = Shape{8, fused && n_groups < 64 ? 1 : 2};
-    else if (units <= 256 && n_groups >= 64) s = Shape{8, 2};
-    else if (units <= 768) s = Shape{4, 2};
-    else if (units <= 1536 && fused && n_groups <= 64) s = Shape{2, 2};
-    else if (units > 2048 && !fused && n_groups >= 32) s = Shape{4, 2};
+//
+// Grouped queries, an even number a kv head, from 257 units on: 2 or 4 of
+// them share a workgroup, 8 waves of it up to 512 units, 4 up to 1536 (1280
+// units of 64 groups: 27.8 us with 2 heads x 2 waves, 33.8 with 4 x 1, 36.4
+// one head a workgroup; 512: 14.5 with 2 x 4, 15.2 with 2 x 2, 17.1).  Past
+// that 4 x 1 (4096: 63.7 against 73.1 with 2 x 2 and 98.0), or with 2 heads
+// a kv head 2 x 2 from 32 groups on (4096 of 64: 71.4, 2 x 1 79.9) and 2 x 1
+// below (4800 of 19: 30.3, 2 x 2 32.0).  8 x 1 gains nothing over 4 x 1.
+constexpr Shape default_shape(int64_t units, int n_groups, int q_per_kv, bool fused) {
+    Shape s{1, 2, 1};
+    if (q_per_kv % 2 == 0 && units > 256 && n_groups > 1) {
+        s = units <= 512 ? Shape{4, 2, 2}
+            : units <= 1536 ? Shape{2, 2, 2}
+            : q_per_kv % 4 == 0 ? Shape{1, 2, 4}
+            : n_groups >= 32 ? Shape{2, 2, 2} : Shape{1, 2, 2};
+    } else if (units < 128) s = Shape{8, fused && n_groups < 64 ? 1 : 2, 1};
+    else if (units <= 256 && n_groups >= 64) s = Shape{8, 2, 1};
+    else if (units <= 768) s = Shape{4, 2, 1};
+    else if (units <= 1536 && fused && n_groups <= 64) s = Shape{2, 2, 1};
+    else if (units > 2048 && !fused && n_groups >= 32) s = Shape{4, 2, 1};
     while (s.nw > 1 && s.nw > n_groups + (fused && n_groups == 1 ? 1 : 0)) s.nw /= 2;
     if (n_groups == 1) s.pf = 1;
     return s;
@@ -761,44 +795,45 @@ constexpr Shape default_shape(int64_t units, int n_groups, bool fused) {
 constexpr bool default_shapes_instantiated() {
     for (int64_t units : {1, 32, 127, 128, 256, 257, 768, 769, 1536, 1537, 2048, 2049, 1 << 20})
         for (int n_groups = 1; n_groups <= 65; ++n_groups)
-            for (bool fused : {false, true})
-                if (!shape_instantiated(default_shape(units, n_groups, fused))) return false;
+            for (int q_per_kv : {1, 2, 3, 4, 6, 8, 16})
+                for (bool fused : {false, true})
+                    if (!shape_instantiated(default_shape(units, n_groups, q_per_kv, fused))) return false;
     return true;
 }
 static_assert(default_shapes_instantiated(), "every default decode shape has a kernel");
 
-// BMO_ATTN_SHAPE = "nw,pf" overrides the default (tuning); a shape without a
-// kernel falls back to one wave with one group in flight.
-Shape pick_shape(int64_t units, int n_groups, bool fused) {
-    Shape s = default_shape(units, n_groups, fused);
+// BMO_ATTN_SHAPE = "nw,pf[,r]" overrides the default (tuning); a shape
+// without a kernel, or with an r that does not divide the query heads of a kv
+// head, falls back to one wave with one group in flight.
+Shape pick_shape(int64_t units, int n_groups, int q_per_kv, bool fused) {
+    Shape s = default_shape(units, n_groups, q_per_kv, fused);
     if (const char *e = std::getenv("BMO_ATTN_SHAPE")) {
-        Shape o{0, 0};
-        if (std::sscanf(e, "%d,%d", &o.nw, &o.pf) == 2) s = o;
+        Shape o{0, 0, 1};
+        if (std::sscanf(e, "%d,%d,%d", &o.nw, &o.pf, &o.r) >= 2) s = o;
     }
+    if (!shape_instantiated(s) || q_per_kv % s.r != 0) s = Shape{1, 1, 1};
     return s;
 }
 
 template <int D>
-bool launch_shape(const DecodeParams &p, bool fused, hipStream_t stream, const Shape &s) {
-#define BMO_SHAPE(NW_, PF_)                                \
-    static_assert(shape_instantiated(Shape{NW_, PF_}));    \
-    if (s.nw == NW_ && s.pf == PF_) {                      \
-        launch_variant<D, NW_, PF_>(p, fused, stream);     \
-        return true;                                       \
-    }
-    BMO_SHAPE(1, 1)
-    BMO_SHAPE(1, 2)
-    BMO_SHAPE(1, 3)
-    BMO_SHAPE(2, 1)
-    BMO_SHAPE(2, 2)
-    BMO_SHAPE(4, 1)
-    BMO_SHAPE(4, 2)
-    BMO_SHAPE(8, 1)
-    BMO_SHAPE(8, 2)
-    BMO_SHAPE(16, 1)
+void launch_shape(const DecodeParams &p, bool fused, hipStream_t stream, const Shape &s) {
+#define BMO_SHAPE(NW_, PF_, R_)                              \
+    static_assert(shape_instantiated(Shape{NW_, PF_, R_}));  \
+    if (s.nw == NW_ && s.pf == PF_ && s.r == R_) return launch_variant<D, NW_, PF_, R_>(p, fused, stream);
+    BMO_SHAPE(1, 1, 1)
+    BMO_SHAPE(1, 2, 1)
+    BMO_SHAPE(2, 1, 1)
+    BMO_SHAPE(2, 2, 1)
+    BMO_SHAPE(4, 1, 1)
+    BMO_SHAPE(4, 2, 1)
+    BMO_SHAPE(8, 1, 1)
+    BMO_SHAPE(8, 2, 1)
+    BMO_SHAPE(1, 2, 2)
+    BMO_SHAPE(2, 2, 2)
+    BMO_SHAPE(4, 2, 2)
+    BMO_SHAPE(1, 2, 4)
 #undef BMO_SHAPE
-    static_assert(sizeof(kShapes) / sizeof(kShapes[0]) == 10, "kShapes lists the shapes dispatched above");
-    return false;
+    static_assert(sizeof(kShapes) / sizeof(kShapes[0]) == 12, "kShapes lists the shapes dispatched above");
 }
 
 }  // namespace
@@ -808,19 +843,17 @@ bool launch_decode(const DecodeParams &params, bool fused, hipStream_t stream) {
     if (units <= 0) return true;
     DecodeParams p = params;
     p.q_per_kv = p.n_heads / p.n_kv;
-    p.div_heads = make_fastdiv((uint32_t) p.n_heads);
     p.layer_base = p.base + p.g.stripe_offset(p.layer, 0, 0);
     p.layer_bytes = p.g.n_groups * p.g.group_stride;
     p.div_qkv = make_fastdiv((uint32_t) p.q_per_kv);
     p.div_ctx = make_fastdiv((uint32_t) p.g.n_ctx);
-    const Shape s = pick_shape(units, p.g.n_groups, fused);
-    if (p.g.head_dim == 128) {
-        if (!launch_shape<128>(p, fused, stream, s)) launch_variant<128, 1, 1>(p, fused, stream);
-    } else if (p.g.head_dim == 64) {
-        if (!launch_shape<64>(p, fused, stream, s)) launch_variant<64, 1, 1>(p, fused, stream);
-    } else {
+    const Shape s = pick_shape(units, p.g.n_groups, p.q_per_kv, fused);
+    if (p.g.head_dim == 128)
+        launch_shape<128>(p, fused, stream, s);
+    else if (p.g.head_dim == 64)
+        launch_shape<64>(p, fused, stream, s);
+    else
         return false;
-    }
     return true;
 }
 

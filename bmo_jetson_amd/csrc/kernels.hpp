@@ -73,10 +73,12 @@ struct DecodeParams {
     int rope;            // nonzero: rotate q (and the fused k_new) by interleaved RoPE at pos
     double rope_r;       // theta^(-2/head_dim): pair i turns by pos * rope_r^i
     // set by launch_decode: the first layer's group 0, the bytes of a layer,
-    // n_heads / n_kv and dividers by n_heads, by n_heads / n_kv and by g.n_ctx
+    // n_heads / n_kv, the query-head sets of an entry (one workgroup each) and
+    // dividers by that number, by n_heads / n_kv and by g.n_ctx
     uint8_t *layer_base;
     int64_t layer_bytes;
     int q_per_kv;
+    int heads_r;
     FastDiv div_heads, div_qkv, div_ctx;
 };
 

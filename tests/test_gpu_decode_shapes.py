@@ -48,7 +48,18 @@ def test_default_shapes(gpu, n_batch, heads, n_ctx, fused):
 
 
 @pytest.mark.parametrize("fused", [False, True])
-@pytest.mark.parametrize("shape", ["2,1", "2,2", "4,2", "8,2"])
+@pytest.mark.parametrize("heads,kv", [(8, 4), (12, 3), (16, 2), (12, 2), (9, 3)])
+@pytest.mark.parametrize("d,n_ctx,n_batch", [(64, 40, 33), (128, 40, 70), (64, 8, 70), (128, 600, 200),
+                                             (64, 500, 200)])
+def test_grouped_queries(gpu, heads, kv, d, n_ctx, n_batch, fused):
+    """2, 4, 8, 6 and 3 query heads a kv head on both sides of the grouped
+    shapes' lines (256, 512 and 1536 units, 32 groups)."""
+    pos = [(n_ctx + 5 * s) if s % 3 else (7 * s) % n_ctx for s in range(n_batch)]
+    _check(gpu, n_batch, heads, kv, d, n_ctx, pos, fused, f"{heads}/{kv} heads, {n_batch} entries")
+
+
+@pytest.mark.parametrize("fused", [False, True])
+@pytest.mark.parametrize("shape", ["2,1", "2,2", "4,2", "8,2", "1,2,2", "2,2,2", "4,2,2"])
 @pytest.mark.parametrize("d,n_ctx,pos", [(128, 512, 700), (128, 512, 20), (128, 3000, 3100), (64, 8, 5),
                                          (128, 100, 95), (64, 200, 450)])
 def test_forced_shapes(gpu, monkeypatch, shape, d, n_ctx, pos, fused):

@@ -363,7 +363,13 @@ int bmo::ring_decode_call(bmo_kv_ring_t *r, const char *fn, bool fused, const bm
         DeviceGuard dg(r->device);
         bmo::DecodeParams p{};
         p.rope = c.rope_theta != 0.0f;
-        p.rope_r = p.rope ? std::pow((double) c.rope_theta, -2.0 / (double) r->g.head_dim) : 0.0;
+        if (p.rope) {
+            double x = std::pow((double) c.rope_theta, -2.0 / (double) r->g.head_dim);
+            for (double &f : p.rope_pow) {
+                f = x;
+                x *= x;
+            }
+        }
         p.base = r->mem;
         p.g = r->g;
         p.layer = c.layer;

@@ -185,22 +185,52 @@ struct Scorer {
     }
 };
 
+// Sine and cosine of a (|a| < 2^31) in double, about 1e-16 off: Cody and
+// Waite's reduction by multiples of pi/2 in three parts (the first fma is
+// exact: a and k pi1 are multiples of 2^-52, their difference below 1), then
+// Taylor polynomials on [-pi/4, pi/4], whose first omitted terms are below
+// 1e-18.  Every lane takes the same instructions: the general library
+// function with its large-argument branch held RoPE's first group back by
+// 0.6 us a launch at B = 1.
+__device__ __forceinline__ void sincos_reduced(double a, double &sn, double &cs) {
+    const double k = __builtin_rint(a * 0.6366197723675814);  // 2 / pi
+    double r = __builtin_fma(-k, 1.5707963267948966, a);
+    r = __builtin_fma(-k, 6.123233995736766e-17, r);
+    r = __builtin_fma(k, 1.4973849048591833e-33, r);
+    const double z = r * r;
+    constexpr double S[8] = {-1.0 / 6.0, 1.0 / 120.0, -1.0 / 5040.0, 1.0 / 362880.0, -1.0 / 39916800.0,
+                             1.0 / 6227020800.0, -1.0 / 1307674368000.0, 1.0 / 355687428096000.0};
+    constexpr double C[8] = {1.0 / 24.0, -1.0 / 720.0, 1.0 / 40320.0, -1.0 / 3628800.0, 1.0 / 479001600.0,
+                             -1.0 / 87178291200.0, 1.0 / 20922789888000.0, -1.0 / 6402373705728000.0};
+    double ps = S[7], pc = C[7];
+#pragma unroll
+    for (int i = 6; i >= 0; --i) {
+        ps = __builtin_fma(ps, z, S[i]);
+        pc = __builtin_fma(pc, z, C[i]);
+    }
+    const double s0 = __builtin_fma(r * z, ps, r);
+    const double c0 = __builtin_fma(z, __builtin_fma(z, pc, -0.5), 1.0);
+    const int q = (int) k;
+    sn = q & 1 ? c0 : s0;
+    cs = q & 1 ? s0 : c0;
+    sn = q & 2 ? -sn : sn;
+    cs = (q + 1) & 2 ? -cs : cs;
+}
+
 // Interleaved RoPE (src/bmo_cuda_kernels.cu:317-354): pair (x[2i], x[2i+1])
 // of a head turns by pos * theta^(-2i/head_dim).  Lane i < D/2 of a wave
-// writes cos and sin (fp32) of pair i to tab: the frequency r^i by binary
-// powers of r = theta^(-2/D) and the angle, cosine and sine in double, so
-// the table is the exact rotation rounded once (the reference evaluates it
-// with fp32 fast intrinsics).
+// writes cos and sin (fp32) of pair i to tab: the frequency r^i as the
+// product of the powers r^(2^k) of i's bits, lowest first, and the angle,
+// cosine and sine in double, so the table is the exact rotation rounded once
+// (the reference evaluates it with fp32 fast intrinsics).
 template <int D>
-__device__ __forceinline__ void rope_table(int pos, double r, int lane, float2 *tab) {
+__device__ __forceinline__ void rope_table(int pos, const double (&pow2)[6], int lane, float2 *tab) {
     if (lane < D / 2) {
-        double f = 1.0, b = r;
-        for (int i = lane; i; i >>= 1) {
-            if (i & 1) f *= b;
-            b *= b;
-        }
+        double f = 1.0;
+#pragma unroll
+        for (int k = 0; k < (D == 128 ? 6 : 5); ++k) f *= (lane >> k) & 1 ? pow2[k] : 1.0;
         double sn, cs;
-        sincos((double) pos * f, &sn, &cs);
+        sincos_reduced((double) pos * f, sn, cs);
         tab[lane] = make_float2((float) cs, (float) sn);
     }
 }
@@ -357,7 +387,7 @@ __global__ __launch_bounds__(64 * R * S) void decode_kernel(DecodeParams p) {
     __shared__ float s_m[NW];
     __shared__ float s_l[NW];
     __shared__ float s_sq[NW][4];
-    __shared__ float2 s_rope[NW][D / 2];
+    __shared__ float2 s_rope[FUSED ? NW : 1][D / 2];
 
     const int lane = threadIdx.x & 63;
     // Wave-uniform where that measured faster (frame 202 against 206 us, 64
@@ -456,8 +486,15 @@ __global__ __launch_bounds__(64 * R * S) void decode_kernel(DecodeParams p) {
 #pragma unroll
         for (int j = 0; j < NB - 1; ++j) load_clamped(j, buf[j]);
     }
-    if (p.rope) rope_table<D>(pos, p.rope_r, lane, s_rope[wave]);  // wave-private LDS
-    prep_digits<D>(q_lo, q_hi, p.qscale, lane, s_dig[wave], s_sq[wave], p.rope ? s_rope[wave] : nullptr);
+    // (only the fused calls rotate)
+    const float2 *rope = nullptr;
+    if constexpr (FUSED) {
+        if (p.rope) {
+            rope_table<D>(pos, p.rope_pow, lane, s_rope[wave]);  // wave-private LDS
+            rope = s_rope[wave];
+        }
+    }
+    prep_digits<D>(q_lo, q_hi, p.qscale, lane, s_dig[wave], s_sq[wave], rope);
     __syncthreads();
     Scorer score;
 #pragma unroll

@@ -71,7 +71,7 @@ struct DecodeParams {
     float *out;          // [n_layers][n_batch][n_heads][head_dim]
     float qscale;        // softmax scale * log2(e)
     int rope;            // nonzero: rotate q (and the fused k_new) by interleaved RoPE at pos
-    double rope_r;       // theta^(-2/head_dim): pair i turns by pos * rope_r^i
+    double rope_pow[6];  // r^(2^k), r = theta^(-2/head_dim): pair i turns by pos * r^i
     // set by launch_decode: the first layer's group 0, the bytes of a layer,
     // n_heads / n_kv, the query-head sets of an entry (one workgroup each) and
     // dividers by that number, by n_heads / n_kv and by g.n_ctx

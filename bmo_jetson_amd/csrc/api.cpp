@@ -380,7 +380,7 @@ int bmo::ring_decode_call(bmo_kv_ring_t *r, const char *fn, bool fused, const bm
         p.session_ids = c.session_ids;
         p.session0 = c.session0;
         p.pos = c.pos;
-        p.pos_scalar = c.pos_host;
+        p.pos_scalar = c.pos ? c.pos_add : c.pos_host;
         p.pos_out = c.pos_out;
         p.pos_out_value = c.pos_out_value;
         p.q = c.q;
@@ -769,7 +769,7 @@ void bmo_launch_decode_attention(const float *q_dev, const float *k_dev, const f
     p.n_heads = n_heads;
     p.n_kv = n_kv_heads;
     p.pos = pos_dev;
-    p.pos_scalar = n_past;
+    p.pos_scalar = pos_dev ? 0 : n_past;
     p.q = q_dev;
     p.k_new = k_dev;
     p.v_new = v_dev;

@@ -470,7 +470,7 @@ __global__ __launch_bounds__(64 * R * S) void decode_kernel(DecodeParams p) {
             }
         }
     }
-    const int pos = p.pos ? p.pos[b] : p.pos_scalar;
+    const int pos = (p.pos ? p.pos[b] : 0) + p.pos_scalar;
     if (p.pos_out && unit == 0 && threadIdx.x == 0) *p.pos_out = p.pos_out_value;
     if (!sid_ok || pos < 0) {
         if (ws == 0)

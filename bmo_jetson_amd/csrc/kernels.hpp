@@ -61,8 +61,8 @@ struct DecodeParams {
                              // (g.n_kv_heads is the allocated head count per stripe set)
     const int *session_ids;  // device, or nullptr -> entry b is session session0 + b
     int session0;
-    const int *pos;          // device [n_batch], or nullptr -> pos_scalar
-    int pos_scalar;
+    const int *pos;          // device [n_batch], nullable: entry b is at pos[b] + pos_scalar,
+    int pos_scalar;          // or at pos_scalar
     int *pos_out;            // nullable: receives pos_out_value (a position the host knows;
     int pos_out_value;       // no workgroup of the launch may read it)
     const float *q;      // [n_layers][n_batch][n_heads][head_dim]
@@ -159,6 +159,7 @@ struct DecodeCall {
     const int *session_ids = nullptr;  // nullptr: entry b is session session0 + b
     int session0 = 0;
     const int *pos = nullptr;          // device; nullptr: every entry is at pos_host
+    int pos_add = 0;                   // added to device positions
     int pos_host = -1;
     int *pos_out = nullptr;
     int pos_out_value = 0;

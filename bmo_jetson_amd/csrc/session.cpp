@@ -1,8 +1,8 @@
 // session.cpp -- the per-session handle of include/bmo_attn.h: the attention
 // part of the reference's bmo_handle (src/bmo_api.cpp:164-172).  A handle
 // owns one session of a ring, a non-blocking HIP stream, a device-resident
-// position that every launch reads (the reference's pos_dev), and a mutex
-// that serializes its calls (src/bmo_api.cpp:28, :415).
+// position (the reference's pos_dev), and a mutex that serializes its calls
+// (src/bmo_api.cpp:28, :415).
 //
 // Two granularities.  A whole token step (forward) runs the fused append +
 // attention of every layer at one position and then advances the position
@@ -13,8 +13,8 @@
 // layer at a time (begin_step, layer, end_step), asynchronously.  Either can
 // be captured into a HIP graph and replayed per token: capture_begin /
 // capture_end bracket whatever the caller enqueues on the handle's stream,
-// and the graph reads the position from device memory, so replays keep
-// attending (and rotating, with RoPE) at the current position.  A capture
+// and the graph reads the position it begins at from device memory, so
+// replays keep attending (and rotating, with RoPE) at the current position.  A capture
 // may start with an asynchronous reset (the depformer's per-frame reset,
 // src/bmo_api.cpp:682) and hold several steps (its 8 codebook steps).  This
 // is what bmo_capture_graphs / bmo_has_cuda_graphs stand for
@@ -42,8 +42,8 @@ struct bmo_attn_session {
     float rope_theta = 0.0f;  // 0: no RoPE
     int device = 0;
     hipStream_t stream = nullptr;
-    int *dev = nullptr;   // dev[0]: position read by every launch; dev[1]: the session id
-    int64_t pos = 0;      // next position; dev[0] holds it once queued work has run
+    int *dev = nullptr;   // the device position
+    int64_t pos = 0;      // next position; *dev holds it once queued work has run
     // what replay runs: a captured step (its buffers), or a recorded graph
     bool step_set = false;
     const float *step_q = nullptr, *step_k = nullptr, *step_v = nullptr;
@@ -99,22 +99,40 @@ void drop_graph(bmo_attn_session_t *s) {
     s->graph = nullptr;
 }
 
-// Queues one layer's fused append + attention at the device position.
-// Allocates nothing and synchronizes nothing, so it can be captured.
+// Queues one layer's fused append + attention at the device position, or
+// inside a capture at the position its step has there: the device position
+// when the replay begins plus the steps recorded before, or, after a reset,
+// their number alone, which the launch then carries itself (the kernel waits
+// for no load of it, and a step's end records nothing: the depformer's frame
+// of 8 steps x 6 layers 203 -> 189 us).  Allocates nothing and synchronizes
+// nothing, so it can be captured.
 int enqueue_layer(bmo_attn_session_t *s, int l, const float *q, const float *k, const float *v,
                   float *out, const char *fn) {
-    const int rc = s->rope_theta > 0.0f
-                       ? bmo_kv_ring_append_decode_rope(s->ring, l, 1, s->dev + 1, s->dev, s->n_heads, q, k,
-                                                        v, out, s->scale, s->rope_theta, s->stream)
-                       : bmo_kv_ring_append_decode(s->ring, l, 1, s->dev + 1, s->dev, s->n_heads, q, k, v,
-                                                   out, s->scale, s->stream);
-    if (rc != BMO_ATTN_OK) return fail(s, rc, ring_message(fn));
+    bmo::DecodeCall c;
+    c.layer = l;
+    c.session0 = s->session;
+    if (s->capturing && s->cap_resets) {
+        c.pos_host = s->cap_adv;
+    } else {
+        c.pos = s->dev;
+        c.pos_add = s->capturing ? s->cap_adv : 0;
+    }
+    c.n_heads = s->n_heads;
+    c.q = q;
+    c.k_new = k;
+    c.v_new = v;
+    c.out = out;
+    c.scale = s->scale;
+    c.rope_theta = s->rope_theta;
+    c.stream = s->stream;
+    const char *call = s->rope_theta > 0.0f ? "bmo_kv_ring_append_decode_rope" : "bmo_kv_ring_append_decode";
+    if (int rc = bmo::ring_decode_call(s->ring, call, true, c)) return fail(s, rc, ring_message(fn));
     return BMO_ATTN_OK;
 }
 
-// Queues the position advance that ends a step.
-int enqueue_advance(bmo_attn_session_t *s, const char *fn) {
-    bmo::launch_advance(s->dev, 1, 1, s->stream);
+// Queues an advance of the device position by n.
+int enqueue_advance(bmo_attn_session_t *s, int n, const char *fn) {
+    bmo::launch_advance(s->dev, 1, n, s->stream);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return fail(s, BMO_ATTN_ERR_HIP, std::string(fn) + ": " + hipGetErrorString(e));
     return BMO_ATTN_OK;
@@ -262,11 +280,8 @@ bmo_attn_session_t *bmo_attn_session_create(bmo_kv_ring_t *ring, int session, in
         s->device = attr.device;
         DeviceGuard dg(s->device);
         hipError_t e = hipStreamCreateWithFlags(&s->stream, hipStreamNonBlocking);
-        if (e == hipSuccess) e = hipMalloc(&s->dev, 2 * sizeof(int));
-        if (e == hipSuccess) {
-            bmo::launch_set_pos(s->dev, 0, s->stream);
-            e = hipMemcpyAsync(s->dev + 1, &s->session, sizeof(int), hipMemcpyHostToDevice, s->stream);
-        }
+        if (e == hipSuccess) e = hipMalloc(&s->dev, sizeof(int));
+        if (e == hipSuccess) bmo::launch_set_pos(s->dev, 0, s->stream);
         if (e == hipSuccess) e = hipGetLastError();
         if (e == hipSuccess) e = hipStreamSynchronize(s->stream);
         if (e != hipSuccess) {
@@ -463,14 +478,12 @@ int bmo_attn_session_end_step(bmo_attn_session_t *s) {
             return fail(s, BMO_ATTN_ERR_ARG, std::string(fn) + ": the position would pass 2^31 - 1");
         }
         DeviceGuard dg(s->device);
-        if (int rc = enqueue_advance(s, fn)) {
-            s->cap_failed = s->capturing;
-            return rc;
-        }
-        if (s->capturing)
-            ++s->cap_adv;
-        else
+        if (s->capturing) {
+            ++s->cap_adv;  // the capture's end records the advances as one
+        } else {
+            if (int rc = enqueue_advance(s, 1, fn)) return rc;
             s->pos = next;
+        }
         s->last_error.clear();
         return BMO_ATTN_OK;
     } catch (...) {
@@ -490,16 +503,13 @@ int bmo_attn_session_reset_async(bmo_attn_session_t *s) {
             s->cap_failed = s->capturing;
             return fail(s, rc, ring_message(fn));
         }
-        bmo::launch_set_pos(s->dev, 0, s->stream);
-        const hipError_t e = hipGetLastError();
-        if (e != hipSuccess) {
-            s->cap_failed = s->capturing;
-            return fail(s, BMO_ATTN_ERR_HIP, std::string(fn) + ": " + hipGetErrorString(e));
-        }
         if (s->capturing) {
             s->cap_resets = true;
             s->cap_adv = 0;
         } else {
+            bmo::launch_set_pos(s->dev, 0, s->stream);
+            const hipError_t e = hipGetLastError();
+            if (e != hipSuccess) return fail(s, BMO_ATTN_ERR_HIP, std::string(fn) + ": " + hipGetErrorString(e));
             s->pos = 0;
         }
         s->last_error.clear();
@@ -551,8 +561,15 @@ int bmo_attn_session_capture_end(bmo_attn_session_t *s) {
     try {
         if (!s->capturing) return fail(s, BMO_ATTN_ERR_ARG, std::string(fn) + ": no capture is open");
         DeviceGuard dg(s->device);
+        // the recorded steps' effect on the device position
+        if (s->cap_resets)
+            bmo::launch_set_pos(s->dev, s->cap_adv, s->stream);
+        else if (s->cap_adv > 0)
+            bmo::launch_advance(s->dev, 1, s->cap_adv, s->stream);
         hipGraph_t graph = nullptr;
-        const hipError_t e = hipStreamEndCapture(s->stream, &graph);
+        hipError_t e = hipGetLastError();
+        const hipError_t ec = hipStreamEndCapture(s->stream, &graph);
+        if (e == hipSuccess) e = ec;
         s->capturing = false;
         if (s->cap_failed) {
             if (graph) (void) hipGraphDestroy(graph);

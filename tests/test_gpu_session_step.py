@@ -80,3 +80,60 @@ def test_overlapping_buffers_run_in_layer_order(gpu):
         check_close(got[layer + 1], ref, f"layer {layer}")
         m.assert_ring_equal(layer, 0)
     sess.close()
+
+
+@pytest.mark.parametrize("resets", ["first", "between", "never"])
+def test_captured_steps_take_their_positions(gpu, resets):
+    """A recorded graph of five steps, with a reset before them, after the
+    second or not at all: each step's layers attend and rotate at the position
+    that the replay's beginning and the steps before them give, and the device
+    position is where an eager step then goes on."""
+    layers, heads, d, n_ctx, steps = 2, 4, 64, 20, 5
+    m = Mirror(gpu, layers, 2, heads, d, n_ctx)
+    for layer in range(layers):
+        m.fill_range(layer, 1, 0, 30, seed=70 + layer)
+    shape = (steps + 1, layers, heads, d)
+    q, k, v = (oracle.normal(80 + i, int(np.prod(shape))).reshape(shape) for i in range(3))
+    qd, kd, vd = m.dev(q), m.dev(k), m.dev(v)
+    out = gpu.full(shape, float("nan"), device="cuda")
+    gpu.cuda.synchronize()
+    sess = Session(m.ring, 1, heads, rope_theta=THETA)
+    reset_at = {"first": 0, "between": 2, "never": None}[resets]
+    sess.capture_begin()
+    for t in range(steps):
+        if t == reset_at:
+            sess.reset_async()
+        for layer in range(layers):
+            sess.layer(layer, qd[t, layer], kd[t, layer], vd[t, layer], out[t, layer])
+        sess.end_step()
+    sess.capture_end()
+
+    def step(t, pos):
+        for layer in range(layers):
+            m.oracle_append(layer, 1, pos, oracle.rope_interleaved(k[t, layer], pos, THETA), v[t, layer])
+            ref = m.oracle_decode(layer, 1, pos, oracle.rope_interleaved(q[t, layer], pos, THETA), heads)
+            check_close(out[t, layer].cpu().numpy(), ref, f"step {t} at {pos}, layer {layer}")
+
+    for start in (30, 41):
+        # a graph with a reset takes no position: its steps before the reset
+        # are at the handle's
+        pos = start if resets == "never" else sess.pos
+        sess.replay(start)
+        for t in range(steps):
+            if t == reset_at:
+                for layer in range(layers):
+                    m.orc[(layer, 1)] = oracle.new_ring(heads, n_ctx, d)
+                pos = 0
+            step(t, pos)
+            pos += 1
+        assert sess.pos == pos
+        for layer in range(layers):  # at the device position the graph left
+            sess.layer(layer, qd[steps, layer], kd[steps, layer], vd[steps, layer], out[steps, layer])
+        sess.end_step()
+        sess.sync()
+        step(steps, pos)
+        assert sess.pos == pos + 1
+    for layer in range(layers):
+        m.assert_ring_equal(layer, 0)
+        m.assert_ring_equal(layer, 1)
+    sess.close()

@@ -22,9 +22,11 @@
 //   prefill_kernel attention over the ring and the staged chunk;
 //   commit_kernel  copies the staged blocks into their ring slots.
 //
-// prefill_kernel: a workgroup of QW waves serves 16*QB*QW queries of one
+// prefill_kernel: a workgroup of QW waves serves 16*QB*QW/KS queries of one
 // (entry, head); each wave owns QB blocks of 16, so every K and V operand it
-// reads from LDS feeds QB matrix instructions.  Keys stream through four LDS
+// reads from LDS feeds QB matrix instructions, or with KS = 2 shares a block
+// with a second wave, each multiplying one of the two tiles of a barrier
+// period, and the two join their sums at the end.  Keys stream through four LDS
 // buffers in tiles of 32 positions: each thread of the loading waves holds
 // its share of the Q4_0 bytes of the next tiles in registers and
 // dequantizes the oldest two into free buffers (K and V row-major); one
@@ -242,9 +244,9 @@ __global__ __launch_bounds__(256) void commit_kernel(PrefillParams p) {
         *reinterpret_cast<const uint32_t *>(src + p.sg.scale_offset(i, blk));
 }
 
-// Launch bounds: 64 * QW threads, one workgroup per CU (QW = 16: four waves
-// per SIMD, at most 128 VGPRs each, which holds the accumulators, the query
-// operands and the fetched tile bytes without spilling).
+// Launch bounds: four waves per SIMD, one workgroup of 16 waves per CU or two
+// of 8, at most 128 VGPRs each, which holds the accumulators, the query
+// operands and the fetched tile bytes without spilling.
 //
 // DIRECT: every (entry, kv head) stripe is read by this one workgroup (one
 // query head per kv head, the whole chunk in one workgroup).  The workgroup
@@ -294,8 +296,8 @@ __device__ uint64_t g_prefill_phases[kPhaseUnits * 16 * kPhaseRec];
     } while (0)
 #endif
 
-template <int D, int QW, int QB, bool DIRECT, bool ALIGNED>
-__global__ __launch_bounds__(64 * QW, QW / 4) void prefill_kernel(PrefillParams p) {
+template <int D, int QW, int QB, int KS, bool DIRECT, bool ALIGNED>
+__global__ __launch_bounds__(64 * QW, 4) void prefill_kernel(PrefillParams p) {
     static_assert(!DIRECT || ALIGNED, "the direct path serves rings of a multiple of 32 slots");
     constexpr int NBLK = D / kQK;
     // LDS rows (fp16) of D + 16 halves, K and V alike: with that stride the
@@ -306,8 +308,8 @@ __global__ __launch_bounds__(64 * QW, QW / 4) void prefill_kernel(PrefillParams 
     // instead of 2.4), on the reads every wave issues right after a barrier.
     constexpr int KROW = D + 16;
     constexpr int VROW = D + 16;
-    constexpr int QWV = 16 * QB;   // queries per wave
-    constexpr int QT = QWV * QW;   // queries per workgroup
+    constexpr int QWV = 16 * QB;        // queries per wave
+    constexpr int QT = QWV * QW / KS;   // queries per workgroup
     constexpr int NT = D / 16;     // output column tiles
     constexpr int NTHR = 64 * QW;
     // dequantization items per tile: (K/V, key, block, 8-byte half)
@@ -321,6 +323,7 @@ __global__ __launch_bounds__(64 * QW, QW / 4) void prefill_kernel(PrefillParams 
     // workgroup synchronize once per TPB tiles.
     constexpr int TPB = 2;
     constexpr int NBUF = 2 * TPB;
+    static_assert(KS == 1 || KS == TPB, "a wave multiplies every tile of a barrier, or one");
     // Blocks whose S^T products are issued together (operands and scales
     // read first): all of them on the direct path; two on the staged path,
     // whose fetch holds more registers (four spill there).
@@ -463,12 +466,11 @@ __global__ __launch_bounds__(64 * QW, QW / 4) void prefill_kernel(PrefillParams 
     // fetch issues its loads (tiles whose keys come from elsewhere -- DIRECT
     // chunk tiles, padding tiles past the end -- read the ring stripe's first
     // slots, which stay cached), so the number of loads in flight is the same
-    // on every path and the compiler's waits stay exact.  Depth: 3 tiles
-    // with 16 waves (4 per SIMD hide the rest; at cfg5 depth 7 measured
-    // 85.7 vs 84.0 us in one earlier build and 78.4 vs 74.2 us in a later
-    // one, where it spilled 3 VGPRs; depth 3 spills in no instantiation), 7
-    // with fewer.
-    constexpr int PF = QW >= 16 ? 3 : 7;
+    // on every path and the compiler's waits stay exact.  Depth: 3 tiles (4
+    // waves per SIMD hide the rest; at cfg5 depth 7 measured 85.7 vs 84.0 us
+    // in one earlier build and 78.4 vs 74.2 us in a later one, where it
+    // spilled 3 VGPRs; depth 3 spills in no instantiation).
+    constexpr int PF = 3;
     static_assert((PF + 1) % NBUF == 0, "the unrolled slot must determine the LDS buffer");
     uint2 raw[PF + 1][IPT];
     uint32_t rawd[PF + 1][IPT];
@@ -499,7 +501,9 @@ __global__ __launch_bounds__(64 * QW, QW / 4) void prefill_kernel(PrefillParams 
             if constexpr (!ALIGNED) {
                 // the ring's slots wrap inside a tile: per-key slot
                 if (ring_t) {
-                    const uint32_t slot = (uint32_t) (slot0 + it_key[j]) % (uint32_t) n_ctx;
+                    uint32_t slot = (uint32_t) (slot0 + it_key[j]);
+                    if (slot >= (uint32_t) n_ctx) slot -= (uint32_t) n_ctx;
+                    if (n_ctx < kTK) slot %= (uint32_t) n_ctx;  // (wave-uniform)
                     const uint32_t row = slot % G;
                     const uint32_t in_row = it_code[j] - (uint32_t) (it_key[j] % G) * (D / 2);
                     gp = ring + (uint64_t) (slot / G) * ring_gs;
@@ -576,7 +580,8 @@ __global__ __launch_bounds__(64 * QW, QW / 4) void prefill_kernel(PrefillParams 
     // zeroed.
     const int n = lane & 15;
     const int c = lane >> 4;
-    const int wq0 = i0 + wave * QWV;  // first query of this wave
+    const int wq0 = i0 + wave / KS * QWV;  // first query of this wave
+    const int wk = wave % KS;              // ... and the tile it takes of each barrier (KS > 1)
     uint2 qlo[QB][NBLK], qhi[QB][NBLK];
     int mrel[QB];  // this lane's query position minus 4c (mask arithmetic)
 #pragma unroll
@@ -956,8 +961,12 @@ __global__ __launch_bounds__(64 * QW, QW / 4) void prefill_kernel(PrefillParams 
                     if (touch_on && base + u == touch_at) touch_successor();
                 }
                 BMO_PHASE_LOOP();
+                if constexpr (KS == 1) {
 #pragma unroll
-                for (int k = 0; k < TPB; ++k) compute((u + k) % NBUF, tile_of(base + u + k));
+                    for (int k = 0; k < TPB; ++k) compute((u + k) % NBUF, tile_of(base + u + k));
+                } else {
+                    compute(u % NBUF + wk, tile_of(base + u + wk));
+                }
             }
         }
     };
@@ -980,6 +989,48 @@ __global__ __launch_bounds__(64 * QW, QW / 4) void prefill_kernel(PrefillParams 
     // such rings take the staged path; it stays as a guard.
     if constexpr (DIRECT)
         if (!has_items) commit_until(p.n_tok);
+
+    // KS: the waves of a query block each hold the softmax state of half the
+    // tiles.  The second hands its sums over in the tile buffers (nobody reads
+    // a tile any more), with each query's offset and weight sum, and the first joins them at the larger offset and stores.
+    if constexpr (KS > 1) {
+        constexpr int XQ = (NT / 2) * 64;  // float4s of half a wave's sums
+        static_assert(QB == 1 && sizeof(sV) >= QW / KS * XQ * sizeof(float4_t) &&
+                          sizeof(sK) >= QW / KS * (XQ * sizeof(float4_t) + 32 * sizeof(float)),
+                      "room for the hand-over");
+        const int qg = wave / KS;
+        float4_t *const xv = reinterpret_cast<float4_t *>(&sV[0][0]) + qg * XQ;
+        float4_t *const xk = reinterpret_cast<float4_t *>(&sK[0][0]) + qg * XQ;
+        float *const xs = reinterpret_cast<float *>(reinterpret_cast<float4_t *>(&sK[0][0]) + QW / KS * XQ) + qg * 32;
+        lds_barrier();
+        if (wk == 1) {
+#pragma unroll
+            for (int t = 0; t < NT / 2; ++t) {
+                xv[t * 64 + lane] = acc[0][t];
+                xk[t * 64 + lane] = acc[0][NT / 2 + t];
+            }
+            // a query that has seen no key is at the floor
+            if (c == 0) xs[n] = dl[0] == 0.0f ? -cneg[0] : kMaxFloor;
+            if (n == 0)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) xs[16 + 4 * c + v] = accl[0][v];
+        }
+        lds_barrier();
+        if (wk == 1) return;
+        const float m0 = dl[0] == 0.0f ? -cneg[0] : kMaxFloor, m1 = xs[n];
+        const float m = fmaxf(m0, m1);
+        const float f0 = __builtin_amdgcn_exp2f(m0 - m), f1 = __builtin_amdgcn_exp2f(m1 - m);
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const float a0 = __shfl(f0, 4 * c + v), a1 = __shfl(f1, 4 * c + v);
+            accl[0][v] = accl[0][v] * a0 + xs[16 + 4 * c + v] * a1;
+#pragma unroll
+            for (int t = 0; t < NT / 2; ++t) {
+                acc[0][t][v] = acc[0][t][v] * a0 + xv[t * 64 + lane][v] * a1;
+                acc[0][NT / 2 + t][v] = acc[0][NT / 2 + t][v] * a0 + xk[t * 64 + lane][v] * a1;
+            }
+        }
+    }
 
     // Every acc row (query 4c + v) divides by its weight sum.  Lane 4qd + j
     // (of the 16 sharing c) holds, for column tile t, element
@@ -1037,27 +1088,82 @@ namespace {
 // matrix latencies overlap another's work.  Against 8 waves x 32 queries
 // (QB = 2, each K/V operand read feeding two matrix instructions, half the
 // LDS reads per query), both on the staged path at cfg5: 92.7-93.0 vs
-// 106.5-106.6 us (ring history full), 60.7 vs 69.1 us (empty); in an
-// earlier build also GQA 4:1, 256 tokens: 84-85 vs 91-94 us; 512-token
-// chunks: 91-93 vs 99-100 us; head_dim 64 GQA 4:1 on an 8-slot ring: 13.9
-// vs 16.7 us.
-// Smaller workgroups for short chunks (4 waves below 129 tokens) were
-// measured slower whenever the ring holds history: the window's tiles
-// dominate, and all waves share their dequantization.
+// 106.5-106.6 us (ring history full), 60.7 vs 69.1 us (empty).
+// Fewer queries a workgroup mean as many tiles to dequantize for less work,
+// so smaller ones pay where 256-query workgroups leave CUs idle: few units,
+// short chunks, a nearly empty last round (below).
 constexpr int kQW = 16;
 constexpr int kQB = 1;
-constexpr int kQT = 16 * kQB * kQW;  // queries per workgroup
+constexpr int kQT = 16 * kQB * kQW;  // queries per workgroup of the direct path
 
-template <int D>
-void launch_attention(const PrefillParams &p, bool direct, dim3 grid, hipStream_t stream) {
+// Workgroup of the staged path: qw waves, ks of them on each block of 16
+// queries.
+struct StagedShape {
+    int qw, ks;
+    constexpr int queries() const { return 16 * kQB * qw / ks; }
+};
+constexpr StagedShape kStagedShapes[] = {{16, 1}, {16, 2}, {8, 1}, {8, 2}};
+
+// The time of a staged call's workgroups in units of one round of 256
+// workgroups of 16 waves x 16 queries, one a CU.  A 16-wave workgroup fills a
+// CU; two 8-wave ones fit, and slow each other down.  Measured with 8 of 32
+// heads' K/V, 1024 slots, 500 and 256 tokens (us; 16 x 1, 16 x 2, 8 x 1, 8 x
+// 2): 1 session 61.7 / 50.2 / 54.9 / 43.8, 2 sessions 62.9 / 51.0 / 56.1 /
+// 59.6, 3 sessions 64.7 / 92.8 / 76.7 / 87.1, 16 x 256 tokens 124 / 178 / 140
+// / 196; 24 sessions x 64 tokens 120.9 / 118.5 / 87.7 / 85.8.
+constexpr double staged_cost(const StagedShape &s, int64_t workgroups) {
+    const int per_cu = s.qw == 16 ? 1 : 2;
+    const double alone = s.qw == 16 ? (s.ks == 1 ? 1.0 : 0.81) : (s.ks == 1 ? 0.88 : 0.71);
+    const double shared = s.ks == 1 ? 1.155 : 0.95;
+    const int64_t round = 256 * per_cu;
+    const int64_t rest = workgroups % round;
+    return (double) (workgroups / round) * (per_cu == 1 ? alone : shared) +
+           (rest == 0 ? 0.0 : rest <= 256 ? alone : shared);
+}
+
+// The cheapest shape; a smaller one only if it saves a twentieth.
+constexpr StagedShape staged_shape(int64_t units, int n_tok) {
+    StagedShape best = kStagedShapes[0];
+    double cost = 0.95 * staged_cost(best, units * ((n_tok + best.queries() - 1) / best.queries()));
+    for (int i = 1; i < 4; ++i) {
+        const StagedShape s = kStagedShapes[i];
+        const double c = staged_cost(s, units * ((n_tok + s.queries() - 1) / s.queries()));
+        if (c < cost) {
+            best = s;
+            cost = c;
+        }
+    }
+    return best;
+}
+static_assert(staged_shape(512, 256).qw == 16 && staged_shape(512, 256).ks == 1, "full rounds: 256 queries");
+static_assert(staged_shape(32, 500).qw == 8 && staged_shape(32, 500).ks == 2, "256 workgroups of 64 queries");
+static_assert(staged_shape(64, 500).qw == 16 && staged_shape(64, 500).ks == 2, "256 workgroups of 128 queries");
+
+template <int D, int QW, int KS, bool DIRECT>
+void launch_attention(const PrefillParams &p, hipStream_t stream) {
+    const int qt = 16 * kQB * QW / KS;
+    const dim3 grid((unsigned) ((int64_t) p.n_batch * p.n_heads * ((p.n_tok + qt - 1) / qt)));
     // ring tiles 32 slots wide never wrap when n_ctx is a multiple of 32
     // (the direct path requires it)
-    if (direct)
-        hipLaunchKernelGGL((prefill_kernel<D, kQW, kQB, true, true>), grid, dim3(64 * kQW), 0, stream, p);
-    else if (p.g.n_ctx % kTK == 0)
-        hipLaunchKernelGGL((prefill_kernel<D, kQW, kQB, false, true>), grid, dim3(64 * kQW), 0, stream, p);
+    if (DIRECT || p.g.n_ctx % kTK == 0)
+        hipLaunchKernelGGL((prefill_kernel<D, QW, kQB, KS, DIRECT, true>), grid, dim3(64 * QW), 0, stream, p);
     else
-        hipLaunchKernelGGL((prefill_kernel<D, kQW, kQB, false, false>), grid, dim3(64 * kQW), 0, stream, p);
+        hipLaunchKernelGGL((prefill_kernel<D, QW, kQB, KS, false, DIRECT>), grid, dim3(64 * QW), 0, stream, p);
+}
+
+template <int D>
+void launch_attention(const PrefillParams &p, bool direct, hipStream_t stream) {
+    const StagedShape s = staged_shape((int64_t) p.n_batch * p.n_heads, p.n_tok);
+    if (direct)
+        launch_attention<D, kQW, 1, true>(p, stream);
+    else if (s.qw == 16 && s.ks == 1)
+        launch_attention<D, 16, 1, false>(p, stream);
+    else if (s.qw == 16)
+        launch_attention<D, 16, 2, false>(p, stream);
+    else if (s.ks == 1)
+        launch_attention<D, 8, 1, false>(p, stream);
+    else
+        launch_attention<D, 8, 2, false>(p, stream);
 }
 
 }  // namespace
@@ -1103,14 +1209,12 @@ bool launch_prefill(const PrefillParams &p, hipStream_t stream) {
         hipLaunchKernelGGL(stage_kernel, dim3((unsigned) ((stage_threads + 255) / 256)), dim3(256), 0,
                            stream, p);
     }
-    const int qt = kQT;
-    const dim3 grid((unsigned) ((int64_t) p.n_batch * p.n_heads * ((p.n_tok + qt - 1) / qt)));
     PrefillParams pa = p;
     pa.n_resident = resident_workgroups();
     if (p.g.head_dim == 128)
-        launch_attention<128>(pa, direct, grid, stream);
+        launch_attention<128>(pa, direct, stream);
     else
-        launch_attention<64>(pa, direct, grid, stream);
+        launch_attention<64>(pa, direct, stream);
     if (!direct) {
         const int commit_threads = p.n_batch * p.n_tok * p.n_kv * nblk;
         hipLaunchKernelGGL(commit_kernel, dim3((unsigned) ((commit_threads + 255) / 256)), dim3(256), 0,

@@ -100,7 +100,10 @@ struct PrefillParams {
     const uint16_t *v;
     float *out;    // [n_batch][n_tok][n_heads][head_dim]
     float qscale;  // softmax scale * log2(e)
-    int n_resident;  // set by launch_prefill: workgroups the device runs at once (0: unknown)
+    // set by launch_prefill: workgroups the device runs at once (0: unknown),
+    // and the first (entry, query head) unit of an attention launch
+    int n_resident;
+    int unit0;
 };
 
 // n_blocks blocks, from block `first` on, of one session's K (which 0) or V

@@ -360,8 +360,9 @@ __global__ __launch_bounds__(64 * QW, 4) void prefill_kernel(PrefillParams p) {
     // (scalars: the divisions run on the vector unit, readfirstlane keeps
     // their results, and the addresses derived from them, in SGPRs)
     const int n_qt = (p.n_tok + QT - 1) / QT;
-    const int unit = __builtin_amdgcn_readfirstlane((int) blockIdx.x / n_qt);
-    const int qt = (int) blockIdx.x - unit * n_qt;
+    const int lunit = __builtin_amdgcn_readfirstlane((int) blockIdx.x / n_qt);  // unit of the launch
+    const int qt = (int) blockIdx.x - lunit * n_qt;
+    const int unit = lunit + p.unit0;
     const int b = __builtin_amdgcn_readfirstlane(unit / p.n_heads);
     const int h = unit - b * p.n_heads;
     const int i0 = qt * QT;
@@ -1135,14 +1136,33 @@ constexpr StagedShape staged_shape(int64_t units, int n_tok) {
     }
     return best;
 }
+// The units that go ahead in full rounds of the first shape, when the rest in
+// a shape of its own then takes a twentieth less in all than every unit in
+// one (0: one launch).  A second launch costs as much as about 0.05 rounds.
+// 160 units of 500 tokens, 320 workgroups of 256 queries: 128 units in one
+// round and 32 in 256 workgroups of 64 queries, XX us against 110.
+constexpr int64_t staged_full_units(int64_t units, int n_tok) {
+    auto cost = [=](int64_t n) {
+        const StagedShape s = staged_shape(n, n_tok);
+        return staged_cost(s, n * ((n_tok + s.queries() - 1) / s.queries()));
+    };
+    const int64_t n_qt = (n_tok + kStagedShapes[0].queries() - 1) / kStagedShapes[0].queries();
+    const int64_t rounds = units * n_qt / 256;
+    const int64_t full = rounds * 256 / n_qt;
+    if (full == 0 || full == units) return 0;
+    return (double) rounds + 0.05 + cost(units - full) < 0.95 * cost(units) ? full : 0;
+}
+static_assert(staged_full_units(160, 500) == 128 && staged_full_units(512, 256) == 0,
+              "a quarter of a round goes apart, full rounds do not");
+
 static_assert(staged_shape(512, 256).qw == 16 && staged_shape(512, 256).ks == 1, "full rounds: 256 queries");
 static_assert(staged_shape(32, 500).qw == 8 && staged_shape(32, 500).ks == 2, "256 workgroups of 64 queries");
 static_assert(staged_shape(64, 500).qw == 16 && staged_shape(64, 500).ks == 2, "256 workgroups of 128 queries");
 
 template <int D, int QW, int KS, bool DIRECT>
-void launch_attention(const PrefillParams &p, hipStream_t stream) {
+void launch_attention(const PrefillParams &p, int64_t units, hipStream_t stream) {
     const int qt = 16 * kQB * QW / KS;
-    const dim3 grid((unsigned) ((int64_t) p.n_batch * p.n_heads * ((p.n_tok + qt - 1) / qt)));
+    const dim3 grid((unsigned) (units * ((p.n_tok + qt - 1) / qt)));
     // ring tiles 32 slots wide never wrap when n_ctx is a multiple of 32
     // (the direct path requires it)
     if (DIRECT || p.g.n_ctx % kTK == 0)
@@ -1151,19 +1171,28 @@ void launch_attention(const PrefillParams &p, hipStream_t stream) {
         hipLaunchKernelGGL((prefill_kernel<D, QW, kQB, KS, false, DIRECT>), grid, dim3(64 * QW), 0, stream, p);
 }
 
+// Attention of units unit0 .. unit0 + units - 1 in one staged shape.
+template <int D>
+void launch_staged(const PrefillParams &params, int64_t unit0, int64_t units, const StagedShape &s, hipStream_t stream) {
+    PrefillParams p = params;
+    p.unit0 = (int) unit0;
+    if (s.qw == 16 && s.ks == 1)
+        launch_attention<D, 16, 1, false>(p, units, stream);
+    else if (s.qw == 16)
+        launch_attention<D, 16, 2, false>(p, units, stream);
+    else if (s.ks == 1)
+        launch_attention<D, 8, 1, false>(p, units, stream);
+    else
+        launch_attention<D, 8, 2, false>(p, units, stream);
+}
+
 template <int D>
 void launch_attention(const PrefillParams &p, bool direct, hipStream_t stream) {
-    const StagedShape s = staged_shape((int64_t) p.n_batch * p.n_heads, p.n_tok);
-    if (direct)
-        launch_attention<D, kQW, 1, true>(p, stream);
-    else if (s.qw == 16 && s.ks == 1)
-        launch_attention<D, 16, 1, false>(p, stream);
-    else if (s.qw == 16)
-        launch_attention<D, 16, 2, false>(p, stream);
-    else if (s.ks == 1)
-        launch_attention<D, 8, 1, false>(p, stream);
-    else
-        launch_attention<D, 8, 2, false>(p, stream);
+    const int64_t units = (int64_t) p.n_batch * p.n_heads;
+    if (direct) return launch_attention<D, kQW, 1, true>(p, units, stream);
+    const int64_t full = staged_full_units(units, p.n_tok);
+    if (full > 0) launch_staged<D>(p, 0, full, kStagedShapes[0], stream);
+    if (full < units) launch_staged<D>(p, full, units - full, staged_shape(units - full, p.n_tok), stream);
 }
 
 }  // namespace

@@ -23,6 +23,7 @@ pytestmark = pytest.mark.gpu
     (5, 32, 2, 160, 100, 130),                            # 160 units, 130 tokens
     (8, 32, 4, 64, 90, 17),                               # 256 units
     (20, 32, 1, 40, 50, 20),                              # 640 units
+    (5, 32, 2, 512, 100, 500),                            # 128 units in a full round, 32 apart
 ])
 def test_staged_shapes(gpu, d, n_batch, heads, kv, n_ctx, pos0, n_tok):
     m = Mirror(gpu, 1, n_batch, kv, d, n_ctx)

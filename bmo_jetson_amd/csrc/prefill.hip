@@ -146,41 +146,23 @@ static_assert(store_layout_matches(), "output float4 layout");
 constexpr uint32_t kXorLoK = 0x64086408u, kXorHiK = 0x54805480u;
 constexpr uint32_t kXorLoV = 0x64006400u, kXorHiV = 0x54005400u;
 
-// Dequantizes code dword w (bytes 4c..4c+3 of a block) with fp16 scale bits
-// d16 (low half) into 8 fp16 values in perm_elem order: (code - 8) * d, the
-// subtraction exact, the product rounded to nearest.  A low nibble n under
-// the fp16 pattern 0x6400 reads 1024 + n; a high nibble, left in place
-// (n << 4) under 0x5400, reads 64 + n, so no shift per nibble is needed.
-// xlo/xhi are those patterns, K's with the stored bit 3 flipped back (the xor
-// touches only nibble bits and the pattern's own, disjoint bits).
-// SCALED false: the codes alone, (code - 8) exactly (d16 unused).
-template <bool SCALED = true>
-__device__ __forceinline__ half8_t dequant_dword(uint32_t w, uint32_t d16, uint32_t xlo, uint32_t xhi) {
+// The codes of dword w (bytes 4c..4c+3 of a block) as 8 fp16 values in
+// perm_elem order: code - 8, exactly.  A low nibble n under the fp16 pattern
+// 0x6400 reads 1024 + n; a high nibble, left in place (n << 4) under 0x5400,
+// reads 64 + n, so no shift per nibble is needed.  xlo/xhi are those patterns,
+// K's with the stored bit 3 flipped back (the xor touches only nibble bits
+// and the pattern's own, disjoint bits).
+__device__ __forceinline__ half8_t dequant_dword(uint32_t w, uint32_t xlo, uint32_t xhi) {
     const half2_t off_lo = {(_Float16) -1032.0f, (_Float16) -1032.0f};
     const half2_t off_hi = {(_Float16) -72.0f, (_Float16) -72.0f};
-    const _Float16 d = __builtin_bit_cast(_Float16, (uint16_t) d16);
-    const half2_t dd = {d, d};
     const uint32_t y = w >> 8;
     half2_t r[4];
     r[0] = __builtin_bit_cast(half2_t, (w & 0x000F000Fu) ^ xlo) + off_lo;
     r[1] = __builtin_bit_cast(half2_t, (y & 0x000F000Fu) ^ xlo) + off_lo;
     r[2] = __builtin_bit_cast(half2_t, (w & 0x00F000F0u) ^ xhi) + off_hi;
     r[3] = __builtin_bit_cast(half2_t, (y & 0x00F000F0u) ^ xhi) + off_hi;
-    if constexpr (SCALED) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) r[i] *= dd;
-    }
     // r[0] = (e0, e2), r[1] = (e1, e3), r[2] = (e16, e18), r[3] = (e17, e19)
-    half8_t o;
-    o[0] = r[0].x;
-    o[1] = r[0].y;
-    o[2] = r[1].x;
-    o[3] = r[1].y;
-    o[4] = r[2].x;
-    o[5] = r[2].y;
-    o[6] = r[3].x;
-    o[7] = r[3].y;
-    return o;
+    return half8_t{r[0].x, r[0].y, r[1].x, r[1].y, r[2].x, r[2].y, r[3].x, r[3].y};
 }
 
 }  // namespace
@@ -446,7 +428,15 @@ __global__ __launch_bounds__(64 * QW, 4) void prefill_kernel(PrefillParams p) {
     static_assert(G % (32 / NBLK) == 0, "a wave's items share a slot group");
     int it_key[IPT], it_grp[IPT];
     bool it_v[IPT];
-    uint32_t it_code[IPT], it_scale[IPT], it_lds[IPT], it_slds[IPT];
+    uint32_t it_code[IPT], it_scale[IPT], it_lds[IPT];
+    // ... what they become: the nibbles' xor patterns, the row piece in LDS
+    // (K and V rows are laid out alike) and the scale's place
+    typedef __attribute__((address_space(3))) _Float16 lds_half;
+    typedef __attribute__((address_space(3))) half8_t lds_half8;
+    static_assert(KROW == VROW, "one row piece offset");
+    uint32_t it_xlo[IPT], it_xhi[IPT];
+    lds_half *it_dst[IPT];
+    int it_kd[IPT];
 #pragma unroll
     for (int j = 0; j < IPT; ++j) {
         const int it = min((int) threadIdx.x + j * NTHR, ITEMS - 1);
@@ -460,7 +450,10 @@ __global__ __launch_bounds__(64 * QW, 4) void prefill_kernel(PrefillParams p) {
         it_code[j] = (uint32_t) ((key % G) * (D / 2) + bb * 16 + which * kVCodeOff + 8 * hf);
         it_scale[j] = (uint32_t) (kScaleOff + ((key % G) * NBLK + bb) * 4);
         it_lds[j] = (uint32_t) (((which * QT + key) * NBLK + bb) * 16 + 8 * hf);
-        it_slds[j] = (uint32_t) ((key * NBLK + bb) * 4);
+        it_xlo[j] = which ? kXorLoV : kXorLoK;
+        it_xhi[j] = which ? kXorHiV : kXorHiK;
+        it_dst[j] = (which ? (lds_half *) &sV[0][0] : (lds_half *) &sK[0][0]) + (key * KROW + bb * kQK + 16 * hf);
+        it_kd[j] = bb * kTK + kd_slot(key);
     }
 
     // Raw tile bytes, fetched PF tiles ahead: this thread's items.  Every
@@ -473,12 +466,19 @@ __global__ __launch_bounds__(64 * QW, 4) void prefill_kernel(PrefillParams p) {
     // spilled 3 VGPRs; depth 3 spills in no instantiation).
     constexpr int PF = 3;
     static_assert((PF + 1) % NBUF == 0, "the unrolled slot must determine the LDS buffer");
+    // The loading waves' own instructions are what a barrier period waits for
+    // (a wave alone issues one every 5 clocks, scalar ones included), so a
+    // tile's place is worked out once, when it is fetched, K and V share one
+    // path to their codes and the loads take scalar bases: 557 -> 373 scalar
+    // and 782 -> 688 vector instructions per four tiles.
     uint2 raw[PF + 1][IPT];
     uint32_t rawd[PF + 1][IPT];
+    int tile[PF + 1];  // ... and the tiles' first positions (a ring tile's is below pos0)
     int f_next = 0;                        // next position in processing order to fetch
     const int r_slot = r_start % n_ctx;    // ring slot of ring tile 0
-    auto fetch = [&](uint2 (&rw)[IPT], uint32_t (&rd)[IPT]) {
+    auto fetch = [&](uint2 (&rw)[IPT], uint32_t (&rd)[IPT], int &t0_out) {
         const int T = tile_of(f_next++);
+        t0_out = tile_t0(T);
         const bool ring_t = T < n_rt;
         // a ring tile's first slot (r_start + 32 T) % n_ctx; 32 T <= n_ctx
         // + 29, so one subtraction suffices when n_ctx is a multiple of 32
@@ -512,6 +512,10 @@ __global__ __launch_bounds__(64 * QW, 4) void prefill_kernel(PrefillParams p) {
                     so = it_scale[j] + (row - (uint32_t) (it_key[j] % G)) * (NBLK * 4);
                 }
             }
+            // (opaque here, so that the loads take a scalar base and a 32-bit
+            // offset: hoisted, the offsets become 64-bit register pairs and
+            // every load a vector addition)
+            asm volatile("" : "+v"(co), "+v"(so));
             rw[j] = *reinterpret_cast<const uint2 *>(gp + co);
             // the whole scale dword: a 16-bit load would be zero-extended
             // into a copy that hipcc places at the loop's back edge, waiting
@@ -519,13 +523,12 @@ __global__ __launch_bounds__(64 * QW, 4) void prefill_kernel(PrefillParams p) {
             rd[j] = *reinterpret_cast<const uint32_t *>(gp + so);
         }
     };
-    // Dequantizes fetched items of tile T into LDS buffer `buf`: K and V
+    // Dequantizes the fetched items of the tile at t0 into LDS buffer `buf`: K and V
     // row-major, the values of code dword cd at slots 8cd..8cd+7 of the block
     // (the order the query operand uses; col_elem maps a column back to its
     // element).
-    auto deposit = [&](int buf, int T, const uint2 (&rw)[IPT], const uint32_t (&rd)[IPT]) {
-        const bool ring_t = T < n_rt;
-        const int t0 = tile_t0(T);
+    auto deposit = [&](int buf, int t0, const uint2 (&rw)[IPT], const uint32_t (&rd)[IPT]) {
+        const bool ring_t = t0 < pos0;
         const int lo = ring_t ? k_lo : pos0;
         const uint32_t span = (uint32_t) ((ring_t ? pos0 - 1 : p_last) - lo);
         // DIRECT chunk tiles: the chunk's blocks in LDS (clamped for padding
@@ -534,39 +537,37 @@ __global__ __launch_bounds__(64 * QW, 4) void prefill_kernel(PrefillParams p) {
 #pragma unroll
         for (int j = 0; j < IPT; ++j) {
             const int it = threadIdx.x + j * NTHR;
-            if (it < ITEMS) {
+            // (the loading waves' last items: a whole wave has one or none)
+            if (IPT == 1 || it < ITEMS) {
                 const int key = it_key[j];
                 const bool live = (uint32_t) (t0 + key - lo) <= span;
                 uint2 w = rw[j];
                 uint32_t sd = rd[j];
                 if constexpr (DIRECT) {
-                    const uint8_t *cp = reinterpret_cast<const uint8_t *>(sCc) + it_lds[j] + coff;
-                    const uint2 cw = *reinterpret_cast<const uint2 *>(cp);
-                    const uint32_t cs = *reinterpret_cast<const uint32_t *>(
-                        reinterpret_cast<const uint8_t *>(sCs) + it_slds[j] + coff / 4);
+                    const uint32_t o = it_lds[j] + coff;
+                    const uint2 cw = *reinterpret_cast<const uint2 *>(reinterpret_cast<const uint8_t *>(sCc) + o);
+                    // the block's scale dword: its place from that of its codes
+                    const uint32_t cs = sCs[(o >> 4) - (it_v[j] ? QT * NBLK : 0)];
                     w = ring_t ? w : cw;
                     sd = ring_t ? sd : cs;
                 }
                 const uint32_t dw = it_v[j] ? sd >> 16 : sd;
                 const uint32_t d16 = live ? dw : 0u;
-                const int bb = (it >> 1) % NBLK;
-                const int hf = it & 1;
-                half8_t v0, v1;
-                _Float16 *dst;
+                // codes (c - 8) for K and V alike; V's times the scale
+                half8_t v0 = dequant_dword(w.x, it_xlo[j], it_xhi[j]);
+                half8_t v1 = dequant_dword(w.y, it_xlo[j], it_xhi[j]);
+                lds_half *const dst = it_dst[j] + buf * (kTK * KROW);
                 if (it_v[j]) {  // (wave-uniform)
-                    v0 = dequant_dword(w.x, d16, kXorLoV, kXorHiV);
-                    v1 = dequant_dword(w.y, d16, kXorLoV, kXorHiV);
-                    dst = &sV[buf][key * VROW + bb * kQK + 16 * hf];
-                } else {
-                    v0 = dequant_dword<false>(w.x, 0u, kXorLoK, kXorHiK);
-                    v1 = dequant_dword<false>(w.y, 0u, kXorLoK, kXorHiK);
-                    dst = &sK[buf][key * KROW + bb * kQK + 16 * hf];
+                    const _Float16 d = __builtin_bit_cast(_Float16, (uint16_t) d16);
+                    v0 *= d;
+                    v1 *= d;
+                } else if ((it & 1) == 0) {
                     // a dead key's scale is 0, so its (finite) block dot
                     // products add nothing before the mask replaces them
-                    if (hf == 0) sKd[buf][bb * kTK + kd_slot(key)] = __builtin_bit_cast(_Float16, (uint16_t) d16);
+                    sKd[buf][it_kd[j]] = __builtin_bit_cast(_Float16, (uint16_t) d16);
                 }
-                *reinterpret_cast<half8_t *>(dst) = v0;
-                *reinterpret_cast<half8_t *>(dst + 8) = v1;
+                *reinterpret_cast<lds_half8 *>(dst) = v0;
+                *reinterpret_cast<lds_half8 *>(dst + 8) = v1;
             }
         }
     };
@@ -609,7 +610,7 @@ __global__ __launch_bounds__(64 * QW, 4) void prefill_kernel(PrefillParams p) {
     if (has_items) {
 #pragma unroll
         for (int j = 0; j < PF; ++j) {
-            fetch(raw[j], rawd[j]);
+            fetch(raw[j], rawd[j], tile[j]);
             __builtin_amdgcn_sched_barrier(0);
         }
     }
@@ -700,9 +701,8 @@ __global__ __launch_bounds__(64 * QW, 4) void prefill_kernel(PrefillParams p) {
         for (int t = 0; t < NT; ++t) acc[qb][t] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
     }
 
-    auto compute = [&](int buf, int T) {
-        const bool ring_t = T < n_rt;
-        const int t0 = tile_t0(T);
+    auto compute = [&](int buf, int t0) {
+        const bool ring_t = t0 < pos0;
         if (wq0 >= p.n_tok || t0 > w_hi || t0 + kTK - 1 < w_lo) return;  // nothing to see
         // S^T for keys 0..15 and 16..31 of the tile: lane l gets keys
         // 4c + v (and 16 + 4c + v) of query n of each query block.  One
@@ -939,10 +939,18 @@ __global__ __launch_bounds__(64 * QW, 4) void prefill_kernel(PrefillParams p) {
 #pragma unroll
             for (int u = 0; u <= PF; u += TPB) {
                 BMO_PHASE_LOOP();
+                // this period's tiles (the loading waves kept them)
+                int now[TPB];
+#pragma unroll
+                for (int k = 0; k < TPB; ++k) {
+                    if constexpr (LOADS)
+                        now[k] = tile[u + k];
+                    else
+                        now[k] = tile_t0(tile_of(base + u + k));
+                }
                 if constexpr (LOADS) {
 #pragma unroll
-                    for (int k = 0; k < TPB; ++k)
-                        deposit((u + k) % NBUF, tile_of(base + u + k), raw[u + k], rawd[u + k]);
+                    for (int k = 0; k < TPB; ++k) deposit((u + k) % NBUF, now[k], raw[u + k], rawd[u + k]);
                     // the next tiles' loads refill the registers just
                     // dequantized; issued before the barrier, they are in
                     // flight while the waves wait (the barrier waits for LDS
@@ -950,7 +958,7 @@ __global__ __launch_bounds__(64 * QW, 4) void prefill_kernel(PrefillParams p) {
 #pragma unroll
                     for (int k = 0; k < TPB; ++k) {
                         const int nxt = (u + k + PF) % (PF + 1);
-                        fetch(raw[nxt], rawd[nxt]);
+                        fetch(raw[nxt], rawd[nxt], tile[nxt]);
                     }
                 }
                 BMO_PHASE_LOOP();
@@ -964,9 +972,9 @@ __global__ __launch_bounds__(64 * QW, 4) void prefill_kernel(PrefillParams p) {
                 BMO_PHASE_LOOP();
                 if constexpr (KS == 1) {
 #pragma unroll
-                    for (int k = 0; k < TPB; ++k) compute((u + k) % NBUF, tile_of(base + u + k));
+                    for (int k = 0; k < TPB; ++k) compute((u + k) % NBUF, now[k]);
                 } else {
-                    compute(u % NBUF + wk, tile_of(base + u + wk));
+                    compute(u % NBUF + wk, wk ? now[1] : now[0]);
                 }
             }
         }

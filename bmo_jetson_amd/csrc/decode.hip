@@ -471,7 +471,8 @@ __global__ __launch_bounds__(64 * R * S) void decode_kernel(DecodeParams p) {
         }
     }
     const int pos = (p.pos ? p.pos[b] : 0) + p.pos_scalar;
-    if (p.pos_out && unit == 0 && threadIdx.x == 0) *p.pos_out = p.pos_out_value;
+    if constexpr (FUSED)
+        if (p.pos_out && unit == 0 && threadIdx.x == 0) *p.pos_out = p.pos_out_value;
     if (!sid_ok || pos < 0) {
         if (ws == 0)
             for (int i = lane; i < D; i += 64) out_row[i] = 0.0f;
@@ -626,11 +627,12 @@ __global__ __launch_bounds__(64 * R * S) void decode_kernel(DecodeParams p) {
     };
     // acc sums w * c with codes 0..15 and the -8 w of every key is owed until
     // the end (csum): over a long run that debt grows past the sums it is
-    // taken from, and their rounding with it.  It is paid every kSettle
-    // passes: 32 adds (error against 64 bits, one wave: 32 groups 6.3e-7
-    // without, 4.9e-7 with; 188 groups 1.3e-6 and 5.5e-7).  Eight waves'
-    // runs are short.
-    constexpr int kSettle = 16 / NB;
+    // taken from, and their rounding with it.  It is paid every 15 groups,
+    // in 32 adds, or once in a one-wave unit's run of up to 40, where twice
+    // costs 0.3 % of the launch (error against 64 bits, one wave: 32 groups
+    // 6.3e-7 without, 5.3e-7 with; 188 groups 1.3e-6 and 5.5e-7).  Eight
+    // waves' runs are short.
+    const int settle_every = S == 1 && n_it <= 40 ? 24 / NB : 16 / NB;
     auto settle = [&]() {
         const float c = (-8.0f / 16777216.0f) * csum;
         const float c_hi = 16.0f * c;
@@ -638,7 +640,7 @@ __global__ __launch_bounds__(64 * R * S) void decode_kernel(DecodeParams p) {
         for (int e = 0; e < 32; ++e) acc[e] += e < 16 ? c : c_hi;
         csum = 0.0f;
     };
-    int settle_in = kSettle;
+    int settle_in = settle_every;
     // Steady state: every load is unconditional, so the wait before a group's
     // compute is for that group's loads only (a conditional prefetch would
     // make the compiler wait for the prefetch as well).  buf[u] holds group
@@ -653,7 +655,7 @@ __global__ __launch_bounds__(64 * R * S) void decode_kernel(DecodeParams p) {
         if constexpr (S < 8) {
             if (--settle_in == 0) {
                 settle();
-                settle_in = kSettle;
+                settle_in = settle_every;
             }
         }
     }

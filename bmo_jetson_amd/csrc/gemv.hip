@@ -286,18 +286,20 @@ __global__ __launch_bounds__(512) void gemv_kernel(GemvParams p) {
 typedef unsigned int u32x4_t __attribute__((ext_vector_type(4)));
 
 // Streaming variant for rows whose byte length is a multiple of 16 (cols a
-// multiple of 256, at most 6144).  A wave owns up to NPOS chunks of two
-// consecutive rows (c0, c0 + stride, ...), at most NPC KiB of contiguous
-// bytes each (4608 bytes at 4096 columns).  Lane l loads the chunk's 16-byte
+// multiple of 256, at most 6144).  A wave owns chunks of two consecutive rows
+// (c0, c0 + stride, ...), at most NPC KiB of contiguous bytes each (4608 bytes
+// at 4096 columns): up to NPOS of them, or with NPOS = kStreamMaxPos any
+// number, that many at a time.  Lane l loads the chunk's 16-byte
 // pieces j * 1024 + 16 l with nontemporal loads (every byte is loaded once,
 // by one lane), the wave copies the chunk into its own LDS area and each
 // lane reads its block pair from there.  One chunk is in flight at a time:
 // the next chunk's loads go out as soon as the current chunk has arrived,
-// before it is multiplied, and the outputs are stored after the last chunk,
-// so that no store enters a wait.  (Against gemv_kernel at cols = 4096:
+// before it is multiplied, and the outputs are stored after the last chunk
+// (of kStreamMaxPos), so that no store enters a wait (but one in four).  (Against gemv_kernel at cols = 4096:
 // more bytes in flight per wave, two chunks or all of them, were measured
 // slower, as were smaller chunks or more workgroups.)
-constexpr int kStreamMaxPos = 4;  // chunks per wave
+constexpr int kStreamMaxPos = 4;  // chunks per wave between stores
+static_assert(kStreamMaxPos % 2 == 0, "chunk k is in buffer k & 1, whatever went before");
 
 __host__ __device__ constexpr size_t gemv_stream_stage_offset(int cols) {
     return ((size_t) cols + (size_t) (cols / 32) * 8 + 15) / 16 * 16;
@@ -321,10 +323,10 @@ __global__ __launch_bounds__(512) void gemv_stream_kernel(GemvParams p) {
     const int row_bytes = nblk * 18;
     const int chunk_bytes = R * row_bytes;
     const int64_t mat_bytes = (int64_t) p.rows * row_bytes;
-    const int n_chunks = (p.rows + R - 1) / R;
+    const int n_chunks = p.rows / R + (p.rows % R != 0);
     const int stride = gridDim.x * (NT / 64);
     const int c0 = blockIdx.x * (NT / 64) + wave;
-    const int n_mine = c0 < n_chunks ? min(NPOS, (n_chunks - 1 - c0) / stride + 1) : 0;
+    const int n_mine = c0 < n_chunks ? (n_chunks - 1 - c0) / stride + 1 : 0;
 
     // chunk k's pieces, unconditionally (so that the waits before the
     // quantization count loads exactly): pieces past the chunk (or the
@@ -332,7 +334,7 @@ __global__ __launch_bounds__(512) void gemv_stream_kernel(GemvParams p) {
     // that are read (rows are a multiple of 16 bytes), and a wave without
     // chunks reads the last chunk
     auto issue = [&](int k, u32x4_t (&w)[NPC]) {
-        const int64_t cbase = (int64_t) min(c0 + k * stride, n_chunks - 1) * chunk_bytes;
+        const int64_t cbase = min((int64_t) c0 + (int64_t) k * stride, (int64_t) n_chunks - 1) * chunk_bytes;
         const int64_t last = min(cbase + chunk_bytes, mat_bytes) - 16;
 #pragma unroll
         for (int j = 0; j < NPC; ++j)
@@ -359,52 +361,54 @@ __global__ __launch_bounds__(512) void gemv_stream_kernel(GemvParams p) {
     XPair xq[NIT];
 #pragma unroll
     for (int i = 0; i < NIT; ++i) xq[i] = load_x_pair(sq, sd, ss, min(lane + 64 * i, npairs - 1));
-    float yv[NPOS][R];
-#pragma unroll
-    for (int k = 0; k < NPOS; ++k) {
-        if (k < n_mine) {  // (wave-uniform)
-            // chunk k is the only one in flight: once it has arrived, the
-            // next goes out (the wait precedes the branch, so that no path
-            // leaves chunk k's registers pending)
-            __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
-            __builtin_amdgcn_sched_barrier(0);
-            if (k + 1 < n_mine) issue(k + 1, wr[(k + 1) & 1]);
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int j = 0; j < NPC; ++j)
-                *reinterpret_cast<u32x4_t *>(stage + j * 1024 + 16 * lane) = wr[k & 1][j];
-#pragma unroll
-            for (int r = 0; r < R; ++r) {
-                float acc = 0.0f;
-#pragma unroll
-                for (int i = 0; i < NIT; ++i) {
-                    const int pr = lane + 64 * i;
-                    if (pr < npairs) {
-                        const uint32_t *src = reinterpret_cast<const uint32_t *>(stage + r * row_bytes + 36 * pr);
-                        uint32_t w[9];
-#pragma unroll
-                        for (int e = 0; e < 9; ++e) w[e] = src[e];
-                        pair_acc(acc, w, xq[i]);
-                    }
-                }
-                yv[k][r] = wave_sum(acc);
-            }
-        }
-    }
-    if (lane == 0) {
+    for (int k0 = 0; k0 < (NPOS == kStreamMaxPos ? n_mine : 1); k0 += NPOS) {
+        float yv[NPOS][R];
 #pragma unroll
         for (int k = 0; k < NPOS; ++k) {
-            const int c = c0 + k * stride;
+            if (k0 + k < n_mine) {  // (wave-uniform)
+                // chunk k0 + k is the only one in flight: once it has
+                // arrived, the next goes out (the wait precedes the branch,
+                // so that no path leaves its registers pending)
+                __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+                __builtin_amdgcn_sched_barrier(0);
+                if (k0 + k + 1 < n_mine) issue(k0 + k + 1, wr[(k + 1) & 1]);
+                __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int r = 0; r < R; ++r)
-                if (k < n_mine && c * R + r < p.rows) p.y[c * R + r] = yv[k][r];
+                for (int j = 0; j < NPC; ++j)
+                    *reinterpret_cast<u32x4_t *>(stage + j * 1024 + 16 * lane) = wr[k & 1][j];
+#pragma unroll
+                for (int r = 0; r < R; ++r) {
+                    float acc = 0.0f;
+#pragma unroll
+                    for (int i = 0; i < NIT; ++i) {
+                        const int pr = lane + 64 * i;
+                        if (pr < npairs) {
+                            const uint32_t *src = reinterpret_cast<const uint32_t *>(stage + r * row_bytes + 36 * pr);
+                            uint32_t w[9];
+#pragma unroll
+                            for (int e = 0; e < 9; ++e) w[e] = src[e];
+                            pair_acc(acc, w, xq[i]);
+                        }
+                    }
+                    yv[k][r] = wave_sum(acc);
+                }
+            }
+        }
+        if (lane == 0) {
+#pragma unroll
+            for (int k = 0; k < NPOS; ++k) {
+                const int64_t row = ((int64_t) c0 + (int64_t) (k0 + k) * stride) * R;
+#pragma unroll
+                for (int r = 0; r < R; ++r)
+                    if (k0 + k < n_mine && row + r < p.rows) p.y[row + r] = yv[k][r];
+            }
         }
     }
 }
 
 template <int NPC, int NIT>
 void launch_stream(const GemvParams &p, int npos, int n_chunks, hipStream_t stream) {
-    const int wgs = (n_chunks + 8 * npos - 1) / (8 * npos);
+    const int wgs = npos > kStreamMaxPos ? 256 : (n_chunks + 8 * npos - 1) / (8 * npos);
     const size_t lds = gemv_stream_stage_offset(p.cols) + (size_t) 8 * NPC * 1024;
     const dim3 grid((unsigned) wgs), block(512);
     if (npos == 1)
@@ -447,15 +451,19 @@ void launch_rows(const GemvParams &p, hipStream_t stream) {
 bool launch_gemv(const GemvParams &p, hipStream_t stream) {
     // Rows of at most 6144 columns whose byte length is a multiple of 16
     // (cols a multiple of 256, so that every piece inside a chunk is loaded
-    // at its own offset), a 16-byte aligned matrix, and up to kStreamMaxPos
-    // two-row chunks per wave of 256 workgroups: the streaming kernel
-    // (BMO_GEMV_STREAM=0 turns it off, for comparison).  Chunks of up to
-    // 4608 bytes take 5 pieces, up to 6912 bytes 7 (56 KB of stages).
-    const int n_chunks = (p.rows + 1) / 2;
-    const int npos = (n_chunks + 256 * 8 - 1) / (256 * 8);
+    // at its own offset) and a 16-byte aligned matrix: the streaming kernel
+    // (BMO_GEMV_STREAM=0 turns it off, for comparison), on at most 256
+    // workgroups of 8 waves.  Chunks of up to 4608 bytes take 5 pieces, up to
+    // 6912 bytes 7 (56 KB of stages).  Past four chunks per wave only rows of
+    // 2048 columns or more: 32000 x 4096 14.6 us against the pair-walking
+    // kernel's 16.5, 30000 x 2048 11.1 / 11.3, but 30000 x 1536 10.75 / 10.6
+    // and 30000 x 1024 10.6 / 10.2, whose chunks are too short for a load of
+    // their own round trip each.
+    const int n_chunks = p.rows / 2 + p.rows % 2;
+    const int npos = (int) (((int64_t) n_chunks + 256 * 8 - 1) / (256 * 8));
     const char *se = std::getenv("BMO_GEMV_STREAM");
     if (p.cols <= 6144 && p.cols % 256 == 0 && (reinterpret_cast<uintptr_t>(p.w) & 15) == 0 &&
-        npos <= kStreamMaxPos && !(se && se[0] == '0')) {
+        (npos <= kStreamMaxPos || p.cols >= 2048) && !(se && se[0] == '0')) {
         if (p.cols <= 4096)
             launch_stream<5, 1>(p, npos, n_chunks, stream);
         else

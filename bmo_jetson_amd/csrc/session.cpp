@@ -92,7 +92,9 @@ std::string ring_message(const char *what) {
     return std::string(what) + ": " + (m && *m ? m : "ring call failed");
 }
 
-void drop_graph(bmo_attn_session_t *s) {
+// Forgets what replay runs, a recorded graph or a captured step.
+void drop_replay(bmo_attn_session_t *s) {
+    s->step_set = false;
     if (s->exec) (void) hipGraphExecDestroy(s->exec);
     if (s->graph) (void) hipGraphDestroy(s->graph);
     s->exec = nullptr;
@@ -205,7 +207,7 @@ int keep_graph(bmo_attn_session_t *s, hipGraph_t graph, bool resets, int adv, co
         (void) hipGraphDestroy(graph);
         return fail(s, BMO_ATTN_ERR_HIP, std::string(fn) + ": instantiate: " + hipGetErrorString(e));
     }
-    drop_graph(s);
+    drop_replay(s);
     s->graph = graph;
     s->exec = exec;
     s->graph_resets = resets;
@@ -313,7 +315,7 @@ void bmo_attn_session_free(bmo_attn_session_t *s) {
             s->capturing = false;
         }
         if (s->stream) (void) hipStreamSynchronize(s->stream);
-        drop_graph(s);
+        drop_replay(s);
         if (s->dev) (void) hipFree(s->dev);
         if (s->stream) (void) hipStreamDestroy(s->stream);
     } catch (...) {
@@ -376,7 +378,7 @@ int bmo_attn_session_capture(bmo_attn_session_t *s, const float *q, const float 
         DeviceGuard dg(s->device);
         const hipError_t e = hipStreamSynchronize(s->stream);
         if (e != hipSuccess) return fail(s, BMO_ATTN_ERR_HIP, std::string(fn) + ": " + hipGetErrorString(e));
-        drop_graph(s);
+        drop_replay(s);
         s->step_set = true;
         s->step_q = q;
         s->step_k = k;

@@ -137,3 +137,49 @@ def test_captured_steps_take_their_positions(gpu, resets):
         m.assert_ring_equal(layer, 0)
         m.assert_ring_equal(layer, 1)
     sess.close()
+
+
+def test_the_latest_capture_is_what_replay_runs(gpu):
+    """A captured step and a recorded graph replace each other, either way
+    round; a failed recording replaces nothing."""
+    layers, heads, d, n_ctx = 2, 4, 64, 20
+    m = Mirror(gpu, layers, 1, heads, d, n_ctx)
+    shape = (2, layers, heads, d)
+    q, k, v = (oracle.normal(90 + i, int(np.prod(shape))).reshape(shape) for i in range(3))
+    qd, kd, vd = m.dev(q), m.dev(k), m.dev(v)
+    out = gpu.full(shape, float("nan"), device="cuda")
+    gpu.cuda.synchronize()
+    sess = Session(m.ring, 0, heads, rope_theta=THETA)
+
+    def record(t):
+        sess.capture_begin()
+        for layer in range(layers):
+            sess.layer(layer, qd[t, layer], kd[t, layer], vd[t, layer], out[t, layer])
+        sess.end_step()
+        sess.capture_end()
+
+    def fail_to_record():
+        sess.capture_begin()
+        with pytest.raises(RuntimeError):
+            sess.layer(layers, qd[0, 0], kd[0, 0], vd[0, 0], out[0, 0])
+        with pytest.raises(RuntimeError):
+            sess.capture_end()
+
+    pos = 0
+    for t, take in [(0, lambda: sess.capture(qd[0], kd[0], vd[0], out[0])),
+                    (0, fail_to_record),
+                    (1, lambda: record(1)),
+                    (1, fail_to_record),
+                    (0, lambda: sess.capture(qd[0], kd[0], vd[0], out[0]))]:
+        take()
+        assert sess.has_graph
+        out.fill_(float("nan"))
+        gpu.cuda.synchronize()
+        sess.replay(pos)
+        check_close(out[t].cpu().numpy(), _step(m, layers, heads, pos, q[t], k[t], v[t]), f"replay at {pos}")
+        assert gpu.isnan(out[1 - t]).all()
+        pos += 1
+        assert sess.pos == pos
+    for layer in range(layers):
+        m.assert_ring_equal(layer, 0)
+    sess.close()

@@ -10,11 +10,12 @@
 // position 0, afterwards it is the whole ring), and softmax does not depend on
 // key order, so keys are visited in slot order.
 //
-// Work decomposition (gfx950, wave64).  A workgroup of NW waves serves one
-// (batch entry, query head) unit; its waves take contiguous pieces of the
-// window.  Batches with many units use one wave per unit, smaller ones 2 to
-// 8 (16 on request) so that enough waves run, merging in LDS (a split across workgroups would have to merge through
-// device-scope atomics, which serialize across the XCDs).  The ring stores
+// Work decomposition (gfx950, wave64).  S waves serve one (batch entry, query
+// head) unit and take contiguous pieces of its window; a workgroup holds one
+// unit, or R query heads of one kv head.  Batches with many units use one
+// wave per unit, smaller ones 2 to 8 so that enough waves run, merging in LDS
+// (a split across workgroups would have to merge through device-scope
+// atomics, which serialize across the XCDs).  The ring stores
 // slots in groups of G = 64 / LPK keys
 // (ring_layout.hpp), LPK = head_dim / 32 blocks per key, so one group is one
 // wave iteration: lane l owns block l % LPK of key l / LPK and fetches its 16

@@ -294,10 +294,11 @@ typedef unsigned int u32x4_t __attribute__((ext_vector_type(4)));
 // by one lane), the wave copies the chunk into its own LDS area and each
 // lane reads its block pair from there.  One chunk is in flight at a time:
 // the next chunk's loads go out as soon as the current chunk has arrived,
-// before it is multiplied, and the outputs are stored after the last chunk
-// (of kStreamMaxPos), so that no store enters a wait (but one in four).  (Against gemv_kernel at cols = 4096:
-// more bytes in flight per wave, two chunks or all of them, were measured
-// slower, as were smaller chunks or more workgroups.)
+// before it is multiplied, and the outputs are stored after the last chunk of
+// kStreamMaxPos, so that at most one wait in four has stores before it.
+// (Against gemv_kernel at cols = 4096: more bytes in flight per wave, two
+// chunks or all of them, were measured slower, as were smaller chunks or more
+// workgroups.)
 constexpr int kStreamMaxPos = 4;  // chunks per wave between stores
 static_assert(kStreamMaxPos % 2 == 0, "chunk k is in buffer k & 1, whatever went before");
 

@@ -630,14 +630,15 @@ __global__ __launch_bounds__(64 * R * S) void decode_kernel(DecodeParams p) {
     // the end (csum): over a long run that debt grows past the sums it is
     // taken from, and their rounding with it.  It is paid, in 32 adds, after
     // so many groups that a split's error against 64 bits is no larger than
-    // that of eight short runs: every 3 groups of two waves (32 groups:
-    // 4.9e-7 paid every 15, 4.4e-7 every 9, 3.8e-7 every 3; eight waves
-    // 4.0e-7; 25.6 us each), every 9 of four waves or of grouped queries,
-    // which are bound by issue (grouped, 32 heads of 8, 1024 slots: 111 us
-    // every 3, 107 every 9), every 6 of a long one-wave run, and once in a
+    // that of eight short runs: every 3 groups of two or four waves (32
+    // groups, two waves: 4.9e-7 paid every 15, 4.4e-7 every 9, 3.8e-7 every
+    // 3; eight waves 4.0e-7; 25.6 us each; four waves: 4.3e-7 every 9, 3.7e-7
+    // every 3, 12 sessions 150.7 and 152.2 us), every 9 of grouped queries,
+    // which are bound by issue (32 heads of 8, 1024 slots: 111 us every 3,
+    // 107 every 9), every 6 of a long one-wave run, and once in a
     // one-wave run of up to 40, where twice costs 0.3 % of the launch (32
     // groups 6.3e-7 without, 5.3e-7 with).  Eight waves' runs are short.
-    const int settle_every = S == 2 && R == 1 ? 1 : S > 1 || R > 1 ? 9 / NB : n_it <= 40 ? 24 / NB : 6 / NB;
+    const int settle_every = S > 1 && R == 1 ? 1 : R > 1 ? 9 / NB : n_it <= 40 ? 24 / NB : 6 / NB;
     auto settle = [&]() {
         const float c = (-8.0f / 16777216.0f) * csum;
         const float c_hi = 16.0f * c;

@@ -362,7 +362,7 @@ int bmo::ring_decode_call(bmo_kv_ring_t *r, const char *fn, bool fused, const bm
             return fail(r, BMO_ATTN_ERR_ARG, std::string(fn) + ": rope_theta must be positive and finite");
         DeviceGuard dg(r->device);
         bmo::DecodeParams p{};
-        p.rope = c.rope_theta != 0.0f;
+        p.rope = c.rope_theta == 0.0f ? 0 : c.rope_theta < 1.0f ? bmo::kRopeWide : 1;
         if (p.rope) {
             double x = std::pow((double) c.rope_theta, -2.0 / (double) r->g.head_dim);
             for (double &f : p.rope_pow) {

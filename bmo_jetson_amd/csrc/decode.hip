@@ -192,7 +192,8 @@ struct Scorer {
 // Taylor polynomials on [-pi/4, pi/4], whose first omitted terms are below
 // 1e-18.  Every lane takes the same instructions: the general library
 // function with its large-argument branch held RoPE's first group back by
-// 0.6 us a launch at B = 1.
+// 0.6 us a launch at B = 1.  (rope_table takes that function where the
+// angles are not below 2^31.)
 __device__ __forceinline__ void sincos_reduced(double a, double &sn, double &cs) {
     const double k = __builtin_rint(a * 0.6366197723675814);  // 2 / pi
     double r = __builtin_fma(-k, 1.5707963267948966, a);
@@ -223,15 +224,20 @@ __device__ __forceinline__ void sincos_reduced(double a, double &sn, double &cs)
 // writes cos and sin (fp32) of pair i to tab: the frequency r^i as the
 // product of the powers r^(2^k) of i's bits, lowest first, and the angle,
 // cosine and sine in double, so the table is the exact rotation rounded once
-// (the reference evaluates it with fp32 fast intrinsics).
+// (the reference evaluates it with fp32 fast intrinsics).  wide: r > 1, so
+// that pos * r^i can be 2^31 or more (up to about 1e47).
 template <int D>
-__device__ __forceinline__ void rope_table(int pos, const double (&pow2)[6], int lane, float2 *tab) {
+__device__ __forceinline__ void rope_table(int pos, const double (&pow2)[6], bool wide, int lane, float2 *tab) {
     if (lane < D / 2) {
         double f = 1.0;
 #pragma unroll
         for (int k = 0; k < (D == 128 ? 6 : 5); ++k) f *= (lane >> k) & 1 ? pow2[k] : 1.0;
+        const double a = (double) pos * f;
         double sn, cs;
-        sincos_reduced((double) pos * f, sn, cs);
+        if (wide)  // (uniform)
+            sincos(a, &sn, &cs);
+        else
+            sincos_reduced(a, sn, cs);
         tab[lane] = make_float2((float) cs, (float) sn);
     }
 }
@@ -492,7 +498,7 @@ __global__ __launch_bounds__(64 * R * S) void decode_kernel(DecodeParams p) {
     const float2 *rope = nullptr;
     if constexpr (FUSED) {
         if (p.rope) {
-            rope_table<D>(pos, p.rope_pow, lane, s_rope[wave]);  // wave-private LDS
+            rope_table<D>(pos, p.rope_pow, p.rope == kRopeWide, lane, s_rope[wave]);  // wave-private LDS
             rope = s_rope[wave];
         }
     }

@@ -49,6 +49,8 @@ inline FastDiv make_fastdiv(uint32_t d) {
     return FastDiv{(uint32_t) m, s};
 }
 
+constexpr int kRopeWide = 2;  // DecodeParams::rope of a theta < 1
+
 struct DecodeParams {
     uint8_t *base;  // ring allocation; the fused path writes the current slot
     RingGeom g;
@@ -70,7 +72,8 @@ struct DecodeParams {
     const float *v_new;
     float *out;          // [n_layers][n_batch][n_heads][head_dim]
     float qscale;        // softmax scale * log2(e)
-    int rope;            // nonzero: rotate q (and the fused k_new) by interleaved RoPE at pos
+    int rope;            // nonzero: rotate q (and the fused k_new) by interleaved RoPE at pos;
+                         // kRopeWide: theta < 1, whose angles can pass every position
     double rope_pow[6];  // r^(2^k), r = theta^(-2/head_dim): pair i turns by pos * r^i
     // set by launch_decode: the first layer's group 0, the bytes of a layer,
     // n_heads / n_kv, the query-head sets of an entry (one workgroup each) and

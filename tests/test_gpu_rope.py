@@ -55,6 +55,16 @@ def test_rope_positions(gpu, pos):
     _step(gpu, m, 0, [(0, pos)], 4, 10000.0, seed=2 + pos % 97)
 
 
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("theta,pos", [(0.5, 3), (0.5, 2**31 - 2), (1e-3, 12_345_678), (1e-30, 97), (1.0, 2**31 - 2)])
+def test_rope_theta_below_one(gpu, d, theta, pos):
+    """Frequencies above 1: angles past 2^31 (up to 1e30 and more), which take
+    the general sine and cosine; theta 1 is the largest angle that does not."""
+    m = Mirror(gpu, 1, 1, 4, d, 64)
+    m.fill_range(0, 0, 0, pos, seed=2500 + pos % 1000)
+    _step(gpu, m, 0, [(0, pos)], 4, float(np.float32(theta)), seed=3 + pos % 97)
+
+
 def test_rope_batched_gqa_and_head_dim_64(gpu):
     m = Mirror(gpu, 2, 5, 2, 128, 96)
     pos = {0: 0, 1: 95, 2: 96, 3: 1234, 4: 77}

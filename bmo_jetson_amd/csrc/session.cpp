@@ -229,11 +229,19 @@ void seek(bmo_attn_session_t *s, int pos) {
     if (pos != s->pos) bmo::launch_set_pos(s->dev, pos, s->stream);
 }
 
+// After a failed call: queues s->pos as the device position again.  The
+// failure may be another call's, found by this one's error check, and what
+// this call queued, the position's new value among it, may run all the same.
+void restore_pos(bmo_attn_session_t *s) { bmo::launch_set_pos(s->dev, (int) s->pos, s->stream); }
+
 // Waits for the queued work; the position is then next_pos.
 int finish(bmo_attn_session_t *s, int64_t next_pos, const char *fn) {
     hipError_t e = hipGetLastError();
     if (e == hipSuccess) e = hipStreamSynchronize(s->stream);
-    if (e != hipSuccess) return fail(s, BMO_ATTN_ERR_HIP, std::string(fn) + ": " + hipGetErrorString(e));
+    if (e != hipSuccess) {
+        restore_pos(s);
+        return fail(s, BMO_ATTN_ERR_HIP, std::string(fn) + ": " + hipGetErrorString(e));
+    }
     s->pos = next_pos;
     s->last_error.clear();
     return BMO_ATTN_OK;
@@ -358,6 +366,7 @@ int bmo_attn_session_forward(bmo_attn_session_t *s, int pos, const float *q, con
         if (int rc = check_pos(s, pos, fn)) return rc;
         DeviceGuard dg(s->device);
         if (int rc = enqueue_step(s, pos, q, k, v, out)) {
+            restore_pos(s);
             (void) hipStreamSynchronize(s->stream);
             return rc;
         }
@@ -408,7 +417,11 @@ int bmo_attn_session_replay(bmo_attn_session_t *s, int pos) {
         if (int rc = check_pos(s, pos, fn)) return rc;
         if (s->step_set) {
             DeviceGuard dg(s->device);
-            if (int rc = enqueue_step(s, pos, s->step_q, s->step_k, s->step_v, s->step_out)) return rc;
+            if (int rc = enqueue_step(s, pos, s->step_q, s->step_k, s->step_v, s->step_out)) {
+                restore_pos(s);
+                (void) hipStreamSynchronize(s->stream);
+                return rc;
+            }
             return finish(s, (int64_t) pos + 1, fn);
         }
         if (!s->graph_resets && (int64_t) pos + s->graph_adv > INT_MAX)
@@ -416,7 +429,10 @@ int bmo_attn_session_replay(bmo_attn_session_t *s, int pos) {
         DeviceGuard dg(s->device);
         if (!s->graph_resets) seek(s, pos);
         const hipError_t e = hipGraphLaunch(s->exec, s->stream);
-        if (e != hipSuccess) return fail(s, BMO_ATTN_ERR_HIP, std::string(fn) + ": " + hipGetErrorString(e));
+        if (e != hipSuccess) {
+            restore_pos(s);
+            return fail(s, BMO_ATTN_ERR_HIP, std::string(fn) + ": " + hipGetErrorString(e));
+        }
         return finish(s, (s->graph_resets ? 0 : (int64_t) pos) + s->graph_adv, fn);
     } catch (...) {
         return fail(s, BMO_ATTN_ERR_INTERNAL, std::string(fn) + ": unknown exception");
@@ -433,7 +449,10 @@ int bmo_attn_session_begin_step(bmo_attn_session_t *s, int pos) {
         DeviceGuard dg(s->device);
         seek(s, pos);
         const hipError_t e = hipGetLastError();
-        if (e != hipSuccess) return fail(s, BMO_ATTN_ERR_HIP, std::string(fn) + ": " + hipGetErrorString(e));
+        if (e != hipSuccess) {
+            restore_pos(s);
+            return fail(s, BMO_ATTN_ERR_HIP, std::string(fn) + ": " + hipGetErrorString(e));
+        }
         s->pos = pos;
         s->last_error.clear();
         return BMO_ATTN_OK;
@@ -483,7 +502,10 @@ int bmo_attn_session_end_step(bmo_attn_session_t *s) {
         if (s->capturing) {
             ++s->cap_adv;  // the capture's end records the advances as one
         } else {
-            if (int rc = enqueue_advance(s, 1, fn)) return rc;
+            if (int rc = enqueue_advance(s, 1, fn)) {
+                restore_pos(s);
+                return rc;
+            }
             s->pos = next;
         }
         s->last_error.clear();
@@ -511,7 +533,10 @@ int bmo_attn_session_reset_async(bmo_attn_session_t *s) {
         } else {
             bmo::launch_set_pos(s->dev, 0, s->stream);
             const hipError_t e = hipGetLastError();
-            if (e != hipSuccess) return fail(s, BMO_ATTN_ERR_HIP, std::string(fn) + ": " + hipGetErrorString(e));
+            if (e != hipSuccess) {
+                restore_pos(s);
+                return fail(s, BMO_ATTN_ERR_HIP, std::string(fn) + ": " + hipGetErrorString(e));
+            }
             s->pos = 0;
         }
         s->last_error.clear();

@@ -164,13 +164,9 @@ bool readout(bmo_kv_ring_t *r, int layer, int session, int which, int t0, int n,
     p.blocks = r->readout_dev;
     for (p.first = 0; p.first < total; p.first += p.n_blocks) {
         p.n_blocks = std::min(most, total - p.first);
-        if (to_ring) {
-            each(p.first, r->readout, p.n_blocks);
-            bmo::launch_import(p, nullptr);
-        } else {
-            bmo::launch_export(p, nullptr);
-        }
-        if (hipGetLastError() != hipSuccess || hipStreamSynchronize(nullptr) != hipSuccess) return false;
+        if (to_ring) each(p.first, r->readout, p.n_blocks);
+        if (bmo::launch_readout(p, to_ring, nullptr) != hipSuccess || hipStreamSynchronize(nullptr) != hipSuccess)
+            return false;
         if (!to_ring) each(p.first, r->readout, p.n_blocks);
     }
     return true;

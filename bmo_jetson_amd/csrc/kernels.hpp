@@ -136,8 +136,8 @@ bool launch_prefill(const PrefillParams &p, hipStream_t stream);
 
 // Bytes of the block buffer of n_blocks blocks: whole workgroups.
 int64_t readout_buffer_bytes(int64_t n_blocks);
-void launch_export(const ReadoutParams &p, hipStream_t stream);
-void launch_import(const ReadoutParams &p, hipStream_t stream);
+// ... returns the launch's own status: no earlier error of the thread counts.
+hipError_t launch_readout(const ReadoutParams &p, bool to_ring, hipStream_t stream);
 
 struct GemvParams {
     const uint8_t *w;  // ggml block_q4_0 rows [rows][cols/32] (18 bytes each)

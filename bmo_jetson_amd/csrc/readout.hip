@@ -84,14 +84,12 @@ int64_t readout_buffer_bytes(int64_t n_blocks) {
     return (n_blocks + kWgBlocks - 1) / kWgBlocks * (kWgBlocks * kBlockBytes);
 }
 
-void launch_export(const ReadoutParams &p, hipStream_t stream) {
+hipError_t launch_readout(const ReadoutParams &p, bool to_ring, hipStream_t stream) {
     const unsigned wgs = (unsigned) ((p.n_blocks + kWgBlocks - 1) / kWgBlocks);
-    hipLaunchKernelGGL(export_kernel, dim3(wgs), dim3(kWgBlocks), 0, stream, p);
-}
-
-void launch_import(const ReadoutParams &p, hipStream_t stream) {
-    const unsigned wgs = (unsigned) ((p.n_blocks + kWgBlocks - 1) / kWgBlocks);
-    hipLaunchKernelGGL(import_kernel, dim3(wgs), dim3(kWgBlocks), 0, stream, p);
+    ReadoutParams arg = p;
+    void *args[] = {&arg};
+    const void *kernel = to_ring ? reinterpret_cast<const void *>(import_kernel) : reinterpret_cast<const void *>(export_kernel);
+    return hipLaunchKernel(kernel, dim3(wgs), dim3(kWgBlocks), args, 0, stream);
 }
 
 }  // namespace bmo

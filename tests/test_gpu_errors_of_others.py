@@ -1,6 +1,7 @@
 """A HIP error that another call of the program left on the thread (here an
 invalid device number, refused on the host).  A handle's call may report it,
-and then neither its position nor where the device goes on has moved."""
+and then neither its position nor where the device goes on has moved; a
+readout neither fails for it nor takes it from the thread."""
 import ctypes
 
 import numpy as np
@@ -16,9 +17,15 @@ pytestmark = pytest.mark.gpu
 THETA = 10000.0
 
 
-def _leave_error():
+def _hip():
     lib()  # its libamdhip64, already loaded
-    assert ctypes.CDLL("libamdhip64.so.7").hipSetDevice(9999) != 0
+    return ctypes.CDLL("libamdhip64.so.7")
+
+
+def _leave_error():
+    error = _hip().hipSetDevice(9999)
+    assert error != 0
+    return error
 
 
 @pytest.mark.parametrize("call", ["forward", "replay", "replay graph", "begin_step", "end_step", "reset_async"])
@@ -71,3 +78,22 @@ def test_a_failed_call_leaves_the_position(gpu, call):
         check_close(out[layer].cpu().numpy(), ref, f"{call}, layer {layer}")
         m.assert_ring_equal(layer, 0)
     sess.close()
+
+
+@pytest.mark.parametrize("n", [5, 40])
+def test_readouts_keep_to_their_own_errors(gpu, n):
+    kv, d, n_ctx = 3, 128, 40
+    m = Mirror(gpu, 1, 2, kv, d, n_ctx)
+    for s in range(2):
+        m.fill_range(0, s, 0, n_ctx, seed=130 + s)
+    gpu.cuda.synchronize()
+    error = _leave_error()
+    blocks = [m.ring.export_q4_0(0, 0, which, 0, n) for which in (0, 1)]
+    k = m.ring.get_k_cache_f32(0, 0, n)
+    for which in (0, 1):
+        m.ring.import_q4_0(0, 1, which, 0, blocks[which])
+        assert np.array_equal(m.ring.export_q4_0(0, 1, which, 0, n), blocks[which])
+        want = m.orc[(0, 0)][which].transpose(1, 0, 2)[:n]
+        assert np.array_equal(blocks[which].reshape(-1), np.ascontiguousarray(want).view(np.uint8).reshape(-1))
+    assert np.array_equal(k, m.ring.get_k_cache_f32(0, 0, n, session=1))
+    assert _hip().hipGetLastError() in (error, 0)  # (0: a runtime that forgets it at the next good call)

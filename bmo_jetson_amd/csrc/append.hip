@@ -93,13 +93,15 @@ __global__ __launch_bounds__(64) void set_pos_kernel(int *pos, int value) {
     if (threadIdx.x == 0) pos[0] = value;
 }
 
-void launch_set_pos(int *pos, int value, hipStream_t stream) {
-    hipLaunchKernelGGL(set_pos_kernel, dim3(1), dim3(64), 0, stream, pos, value);
+hipError_t launch_set_pos(int *pos, int value, hipStream_t stream) {
+    void *args[] = {&pos, &value};
+    return hipLaunchKernel(reinterpret_cast<const void *>(set_pos_kernel), dim3(1), dim3(64), args, 0, stream);
 }
 
-void launch_advance(int *pos, int n, int delta, hipStream_t stream) {
-    hipLaunchKernelGGL(advance_kernel, dim3((unsigned) ((n + 255) / 256)), dim3(256), 0, stream, pos, n,
-                       delta);
+hipError_t launch_advance(int *pos, int n, int delta, hipStream_t stream) {
+    void *args[] = {&pos, &n, &delta};
+    return hipLaunchKernel(reinterpret_cast<const void *>(advance_kernel), dim3((unsigned) ((n + 255) / 256)),
+                           dim3(256), args, 0, stream);
 }
 
 void launch_append(const AppendParams &p, hipStream_t stream) {

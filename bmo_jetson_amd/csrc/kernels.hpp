@@ -125,10 +125,11 @@ struct ReadoutParams {
 };
 
 // Launchers enqueue only; they leave launch errors for the caller's
-// hipGetLastError().  launch_decode returns false for an unsupported head_dim.
+// hipGetLastError(), and those that return a status, their own, return it as
+// well.  launch_decode returns false for an unsupported head_dim.
 void launch_append(const AppendParams &p, hipStream_t stream);
-void launch_advance(int *pos, int n, int delta, hipStream_t stream);
-void launch_set_pos(int *pos, int value, hipStream_t stream);
+hipError_t launch_advance(int *pos, int n, int delta, hipStream_t stream);
+hipError_t launch_set_pos(int *pos, int value, hipStream_t stream);
 bool launch_decode(const DecodeParams &p, bool fused, hipStream_t stream);
 // stage, attend, commit (three kernels in stream order); false for an
 // unsupported head_dim.
@@ -136,7 +137,6 @@ bool launch_prefill(const PrefillParams &p, hipStream_t stream);
 
 // Bytes of the block buffer of n_blocks blocks: whole workgroups.
 int64_t readout_buffer_bytes(int64_t n_blocks);
-// ... returns the launch's own status: no earlier error of the thread counts.
 hipError_t launch_readout(const ReadoutParams &p, bool to_ring, hipStream_t stream);
 
 struct GemvParams {

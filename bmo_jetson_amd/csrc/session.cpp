@@ -134,7 +134,7 @@ int enqueue_layer(bmo_attn_session_t *s, int l, const float *q, const float *k, 
 
 // Queues an advance of the device position by n.
 int enqueue_advance(bmo_attn_session_t *s, int n, const char *fn) {
-    bmo::launch_advance(s->dev, 1, n, s->stream);
+    (void) bmo::launch_advance(s->dev, 1, n, s->stream);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return fail(s, BMO_ATTN_ERR_HIP, std::string(fn) + ": " + hipGetErrorString(e));
     return BMO_ATTN_OK;
@@ -226,13 +226,13 @@ int check_pos(bmo_attn_session_t *s, int pos, const char *fn) {
 // Makes the device position equal pos before the next step (a no-op when the
 // previous step already left it there).
 void seek(bmo_attn_session_t *s, int pos) {
-    if (pos != s->pos) bmo::launch_set_pos(s->dev, pos, s->stream);
+    if (pos != s->pos) (void) bmo::launch_set_pos(s->dev, pos, s->stream);
 }
 
 // After a failed call: queues s->pos as the device position again.  The
 // failure may be another call's, found by this one's error check, and what
 // this call queued, the position's new value among it, may run all the same.
-void restore_pos(bmo_attn_session_t *s) { bmo::launch_set_pos(s->dev, (int) s->pos, s->stream); }
+void restore_pos(bmo_attn_session_t *s) { (void) bmo::launch_set_pos(s->dev, (int) s->pos, s->stream); }
 
 // Waits for the queued work; the position is then next_pos.
 int finish(bmo_attn_session_t *s, int64_t next_pos, const char *fn) {
@@ -291,7 +291,7 @@ bmo_attn_session_t *bmo_attn_session_create(bmo_kv_ring_t *ring, int session, in
         DeviceGuard dg(s->device);
         hipError_t e = hipStreamCreateWithFlags(&s->stream, hipStreamNonBlocking);
         if (e == hipSuccess) e = hipMalloc(&s->dev, sizeof(int));
-        if (e == hipSuccess) bmo::launch_set_pos(s->dev, 0, s->stream);
+        if (e == hipSuccess) (void) bmo::launch_set_pos(s->dev, 0, s->stream);
         if (e == hipSuccess) e = hipGetLastError();
         if (e == hipSuccess) e = hipStreamSynchronize(s->stream);
         if (e != hipSuccess) {
@@ -340,7 +340,7 @@ int bmo_attn_session_reset(bmo_attn_session_t *s) {
         DeviceGuard dg(s->device);
         const int rc = bmo_kv_ring_reset(s->ring, s->session, s->stream);
         if (rc != BMO_ATTN_OK) return fail(s, rc, ring_message(fn));
-        bmo::launch_set_pos(s->dev, 0, s->stream);
+        (void) bmo::launch_set_pos(s->dev, 0, s->stream);
         return finish(s, 0, fn);
     } catch (...) {
         return fail(s, BMO_ATTN_ERR_INTERNAL, std::string(fn) + ": unknown exception");
@@ -531,7 +531,7 @@ int bmo_attn_session_reset_async(bmo_attn_session_t *s) {
             s->cap_resets = true;
             s->cap_adv = 0;
         } else {
-            bmo::launch_set_pos(s->dev, 0, s->stream);
+            (void) bmo::launch_set_pos(s->dev, 0, s->stream);
             const hipError_t e = hipGetLastError();
             if (e != hipSuccess) {
                 restore_pos(s);
@@ -589,12 +589,12 @@ int bmo_attn_session_capture_end(bmo_attn_session_t *s) {
         if (!s->capturing) return fail(s, BMO_ATTN_ERR_ARG, std::string(fn) + ": no capture is open");
         DeviceGuard dg(s->device);
         // the recorded steps' effect on the device position
+        hipError_t e = hipSuccess;
         if (s->cap_resets)
-            bmo::launch_set_pos(s->dev, s->cap_adv, s->stream);
+            e = bmo::launch_set_pos(s->dev, s->cap_adv, s->stream);
         else if (s->cap_adv > 0)
-            bmo::launch_advance(s->dev, 1, s->cap_adv, s->stream);
+            e = bmo::launch_advance(s->dev, 1, s->cap_adv, s->stream);
         hipGraph_t graph = nullptr;
-        hipError_t e = hipGetLastError();
         const hipError_t ec = hipStreamEndCapture(s->stream, &graph);
         if (e == hipSuccess) e = ec;
         s->capturing = false;

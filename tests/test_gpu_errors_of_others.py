@@ -1,7 +1,8 @@
 """A HIP error that another call of the program left on the thread (here an
 invalid device number, refused on the host).  A handle's call may report it,
-and then neither its position nor where the device goes on has moved; a
-readout neither fails for it nor takes it from the thread."""
+and then neither its position nor where the device goes on has moved; the end
+of a recording does not fail for it, and a readout neither fails for it nor
+takes it from the thread."""
 import ctypes
 
 import numpy as np
@@ -77,6 +78,31 @@ def test_a_failed_call_leaves_the_position(gpu, call):
         ref = m.oracle_decode(layer, 0, pos, oracle.rope_interleaved(q[layer], pos, THETA), heads)
         check_close(out[layer].cpu().numpy(), ref, f"{call}, layer {layer}")
         m.assert_ring_equal(layer, 0)
+    sess.close()
+
+
+@pytest.mark.parametrize("reset", [False, True])
+def test_a_recording_ends_whatever_others_left(gpu, reset):
+    heads, d, n_ctx = 4, 64, 40
+    m = Mirror(gpu, 1, 1, heads, d, n_ctx)
+    q, k, v = (oracle.normal(140 + i, heads * d).reshape(heads, d) for i in range(3))
+    qd, kd, vd = m.dev(q), m.dev(k), m.dev(v)
+    out = gpu.full((heads, d), float("nan"), device="cuda")
+    gpu.cuda.synchronize()
+    sess = Session(m.ring, 0, heads, rope_theta=THETA)
+    sess.capture_begin()
+    if reset:
+        sess.reset_async()
+    sess.layer(0, qd, kd, vd, out)
+    sess.end_step()
+    _leave_error()
+    sess.capture_end()
+    assert sess.has_graph
+    _hip().hipGetLastError()
+    sess.replay(0)
+    m.oracle_append(0, 0, 0, oracle.rope_interleaved(k, 0, THETA), v)
+    check_close(out.cpu().numpy(), m.oracle_decode(0, 0, 0, oracle.rope_interleaved(q, 0, THETA), heads))
+    assert sess.pos == 1
     sess.close()
 
 

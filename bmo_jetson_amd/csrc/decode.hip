@@ -808,16 +808,26 @@ constexpr bool shape_instantiated(Shape s) {
 //   1024 units, 3000 slots  72.8 / 70.9 / 67.4 (71.1 / 68.9 / 64.5)
 // Past 2048 units, where one-wave units come in rounds, plain calls take
 // four waves again from 32 groups on (2560 units 32.6 against 34.3 us, 5120
-// 59.5 / 62.9, 3072 38.6 / 38.0; 8 groups, 8192 units: 40.3 / 28.9).  Between 768 and 1536 units two waves win by overlapping the prologues of
-// fused calls on short windows (up to 64 groups), and lose where the window's
-// bytes dominate.  Below 128 units 8 waves: one workgroup a CU at most, and
-// on long windows more waves still pay (3000 slots, 32 units 16.3 against
-// 17.5 us with 4, on 64 or more groups up to 256 units: 128 units 17.6 /
-// 19.0; 32 groups, 32 units, 7.4 / 7.1).  These units' calls are those of a
-// model's layer loop, whose results the next layer quantizes again: their
-// split of the window, and with it every rounding, is the same for all of
-// them.  Fewer groups than waves: fewer waves, but fused one more than the
-// groups, for the new token (depformer frame, one group: 200 / 207 us).
+// 59.5 / 62.9, 3072 38.6 / 38.0; 8 groups, 8192 units: 40.3 / 28.9).
+// Between 768 and 1536 units two waves win by overlapping the prologues of
+// fused calls on short windows (up to 64 groups), and lose where the
+// window's bytes dominate.  Below 128 units 8 waves: one workgroup a CU at
+// most, and on long windows more waves still pay (3000 slots, 32 units 16.3
+// against 17.5 us with 4, on 64 or more groups up to 256 units: 128 units
+// 17.6 / 19.0; 32 groups, 32 units, 7.4 / 7.1).  Fewer groups than waves:
+// fewer waves, but fused one more than the groups, for the new token
+// (depformer frame, one group: 200 / 207 us).
+//
+// units are those of one layer, also where a launch serves several: the
+// split of a unit's window, and with it every rounding of its output, is
+// then that of the layer's call by itself.  With as few waves as leave every
+// unit of the launch resident a step's error against 64 bits grew, since
+// eight short runs round less than four or two longer ones (relative, 8 / 4,
+// 2 or 1 waves: 20 layers of 128 slots 3.4e-7 / 3.7e-7, 64 layers of 512
+// 4.1e-7 / 5.5e-7, 8 kv heads 4.0e-7 / 4.5e-7); 32 layers of 512 slots took
+// 25.5 us then, 28.5 with eight waves.  Eight waves of several layers keep one group
+// in flight each, which changes no result: 32 layers of 512 slots 28.5 us
+// against 34.0, of 3000 slots 80.2 against 84.6.
 //
 // Grouped queries, an even number a kv head, from 257 units on: 2 or 4 of
 // them share a workgroup, 8 waves of it up to 512 units, 4 up to 1536 (1280
@@ -826,7 +836,7 @@ constexpr bool shape_instantiated(Shape s) {
 // that 4 x 1 (4096: 63.7 against 73.1 with 2 x 2 and 98.0), or with 2 heads
 // a kv head 2 x 2 from 32 groups on (4096 of 64: 71.4, 2 x 1 79.9) and 2 x 1
 // below (4800 of 19: 30.3, 2 x 2 32.0).  8 x 1 gains nothing over 4 x 1.
-constexpr Shape default_shape(int64_t units, int n_groups, int q_per_kv, bool fused) {
+constexpr Shape default_shape(int64_t units, int n_layers, int n_groups, int q_per_kv, bool fused) {
     Shape s{1, 2, 1};
     if (q_per_kv % 2 == 0 && units > 256 && n_groups > 1) {
         s = units <= 512 ? Shape{4, 2, 2}
@@ -839,7 +849,7 @@ constexpr Shape default_shape(int64_t units, int n_groups, int q_per_kv, bool fu
     else if (units <= 1536 && fused && n_groups <= 64) s = Shape{2, 2, 1};
     else if (units > 2048 && !fused && n_groups >= 32) s = Shape{4, 2, 1};
     while (s.nw > 1 && s.nw > n_groups + (fused && n_groups == 1 ? 1 : 0)) s.nw /= 2;
-    if (n_groups == 1) s.pf = 1;
+    if (n_groups == 1 || (s.nw == 8 && n_layers > 1)) s.pf = 1;
     return s;
 }
 
@@ -848,7 +858,8 @@ constexpr bool default_shapes_instantiated() {
         for (int n_groups = 1; n_groups <= 65; ++n_groups)
             for (int q_per_kv : {1, 2, 3, 4, 6, 8, 16})
                 for (bool fused : {false, true})
-                    if (!shape_instantiated(default_shape(units, n_groups, q_per_kv, fused))) return false;
+                    for (int n_layers : {1, 2})
+                        if (!shape_instantiated(default_shape(units, n_layers, n_groups, q_per_kv, fused))) return false;
     return true;
 }
 static_assert(default_shapes_instantiated(), "every default decode shape has a kernel");
@@ -856,8 +867,8 @@ static_assert(default_shapes_instantiated(), "every default decode shape has a k
 // BMO_ATTN_SHAPE = "nw,pf[,r]" overrides the default (tuning); a shape
 // without a kernel, or with an r that does not divide the query heads of a kv
 // head, falls back to one wave with one group in flight.
-Shape pick_shape(int64_t units, int n_groups, int q_per_kv, bool fused) {
-    Shape s = default_shape(units, n_groups, q_per_kv, fused);
+Shape pick_shape(int64_t units, int n_layers, int n_groups, int q_per_kv, bool fused) {
+    Shape s = default_shape(units, n_layers, n_groups, q_per_kv, fused);
     if (const char *e = std::getenv("BMO_ATTN_SHAPE")) {
         Shape o{0, 0, 1};
         if (std::sscanf(e, "%d,%d,%d", &o.nw, &o.pf, &o.r) >= 2) s = o;
@@ -890,15 +901,15 @@ void launch_shape(const DecodeParams &p, bool fused, hipStream_t stream, const S
 }  // namespace
 
 bool launch_decode(const DecodeParams &params, bool fused, hipStream_t stream) {
-    const int64_t units = (int64_t) params.n_layers * params.n_batch * params.n_heads;
-    if (units <= 0) return true;
+    const int64_t units = (int64_t) params.n_batch * params.n_heads;  // of a layer
+    if (units <= 0 || params.n_layers <= 0) return true;
     DecodeParams p = params;
     p.q_per_kv = p.n_heads / p.n_kv;
     p.layer_base = p.base + p.g.stripe_offset(p.layer, 0, 0);
     p.layer_bytes = p.g.n_groups * p.g.group_stride;
     p.div_qkv = make_fastdiv((uint32_t) p.q_per_kv);
     p.div_ctx = make_fastdiv((uint32_t) p.g.n_ctx);
-    const Shape s = pick_shape(units, p.g.n_groups, p.q_per_kv, fused);
+    const Shape s = pick_shape(units, p.n_layers, p.g.n_groups, p.q_per_kv, fused);
     if (p.g.head_dim == 128)
         launch_shape<128>(p, fused, stream, s);
     else if (p.g.head_dim == 64)

@@ -156,9 +156,9 @@ bool step_overlaps(const bmo_attn_session_t *s, const float *q, const float *k, 
 // layer's fused append + attention, the last launch leaving pos + 1 as the
 // device position.  A step's inputs are all there when it begins, so one
 // launch serves every layer: at B = 1 a layer alone fills 32 of the chip's
-// 256 CUs and costs a launch, and the 32 of them took 230 us a step (512
-// slots, RoPE) and 579 us (3000 slots) one after another, against 26 and
-// 77 us in one launch.
+// 256 CUs and costs a launch, and the 32 of them took 231 us a step (512
+// slots, RoPE) and 581 us (3000 slots) one after another, against 28.6 and
+// 80.3 us in one launch, whose outputs are the same bit for bit.
 int enqueue_step(bmo_attn_session_t *s, int pos, const float *q, const float *k, const float *v, float *out) {
     const int64_t qs = (int64_t) s->n_heads * s->head_dim;
     const int64_t ks = (int64_t) s->n_kv * s->head_dim;

@@ -57,6 +57,45 @@ def test_step_of_many_layers(gpu, layers, heads, kv, d, n_ctx, pos):
     sess.close()
 
 
+@pytest.mark.parametrize("layers,heads,kv,d,n_ctx,pos,rope", [
+    (20, 32, 32, 128, 128, 300, True),   # runs of few groups
+    (64, 32, 32, 128, 512, 700, True),   # 2048 units in the launch
+    (32, 32, 8, 128, 512, 90, False),    # grouped queries, a partly filled window
+    (8, 16, 16, 64, 8, 40, True),        # one group
+    (6, 16, 4, 64, 200, 450, True),
+    (2, 32, 32, 128, 1100, 2300, False),  # 69 groups
+    (3, 160, 32, 64, 300, 900, True),    # 160 units a layer: four waves
+    (2, 520, 4, 64, 300, 900, True),     # 520: grouped
+])
+def test_a_step_is_its_layers_bit_for_bit(gpu, layers, heads, kv, d, n_ctx, pos, rope):
+    """The layers of a step in one launch give each output, rounding included,
+    as the layer's call by itself."""
+    m = Mirror(gpu, layers, 1, kv, d, n_ctx)
+    g = gpu.Generator(device="cuda")
+    g.manual_seed(5)
+    n = min(pos, n_ctx)
+    for layer in range(layers):
+        rows = gpu.randn(2, n, kv, d, generator=g, device="cuda")
+        m.ring.write(layer, 0, pos - n, rows[0], rows[1], n_tok=n, stream=m.stream)
+    q, k, v = (gpu.randn(layers, h, d, generator=g, device="cuda") for h in (heads, kv, kv))
+    out = gpu.full(q.shape, float("nan"), device="cuda")
+    gpu.cuda.synchronize()
+    sess = Session(m.ring, 0, heads, rope_theta=THETA if rope else 0.0)
+    sess.begin_step(pos)
+    for layer in range(layers):
+        sess.layer(layer, q[layer], k[layer], v[layer], out[layer])
+    sess.end_step()
+    sess.sync()
+    want = out.cpu().numpy().view(np.uint32)
+    sess.capture(q, k, v, out)
+    for step in (lambda: sess.forward(pos, q, k, v, out), lambda: sess.replay(pos)):
+        out.fill_(float("nan"))
+        gpu.cuda.synchronize()
+        step()
+        assert np.array_equal(out.cpu().numpy().view(np.uint32), want)
+    sess.close()
+
+
 def test_overlapping_buffers_run_in_layer_order(gpu):
     """out one layer behind q in one buffer: layer l + 1's query is layer l's
     output, as in a step whose layers run one after another."""

@@ -779,19 +779,6 @@ void launch_variant(const DecodeParams &params, bool fused, hipStream_t stream) 
         hipLaunchKernelGGL((decode_kernel<D, S, PF, false, R>), grid, block, 0, stream, p);
 }
 
-// BMO_ATTN_SHAPE = "nw,pf[,r]" overrides the default (tuning); a shape
-// without a kernel, or with an r that does not divide the query heads of a kv
-// head, falls back to one wave with one group in flight.
-Shape pick_shape(int64_t units, int n_layers, int n_groups, int q_per_kv, bool fused) {
-    Shape s = default_shape(units, n_layers, n_groups, q_per_kv, fused);
-    if (const char *e = std::getenv("BMO_ATTN_SHAPE")) {
-        Shape o{0, 0, 1};
-        if (std::sscanf(e, "%d,%d,%d", &o.nw, &o.pf, &o.r) >= 2) s = o;
-    }
-    if (!shape_instantiated(s) || q_per_kv % s.r != 0) s = Shape{1, 1, 1};
-    return s;
-}
-
 template <int D>
 void launch_shape(const DecodeParams &p, bool fused, hipStream_t stream, const Shape &s) {
 #define BMO_SHAPE(NW_, PF_, R_)                              \
@@ -799,18 +786,20 @@ void launch_shape(const DecodeParams &p, bool fused, hipStream_t stream, const S
     if (s.nw == NW_ && s.pf == PF_ && s.r == R_) return launch_variant<D, NW_, PF_, R_>(p, fused, stream);
     BMO_SHAPE(1, 1, 1)
     BMO_SHAPE(1, 2, 1)
+    BMO_SHAPE(1, 3, 1)
     BMO_SHAPE(2, 1, 1)
     BMO_SHAPE(2, 2, 1)
     BMO_SHAPE(4, 1, 1)
     BMO_SHAPE(4, 2, 1)
     BMO_SHAPE(8, 1, 1)
     BMO_SHAPE(8, 2, 1)
+    BMO_SHAPE(16, 1, 1)
     BMO_SHAPE(1, 2, 2)
     BMO_SHAPE(2, 2, 2)
     BMO_SHAPE(4, 2, 2)
     BMO_SHAPE(1, 2, 4)
 #undef BMO_SHAPE
-    static_assert(sizeof(kShapes) / sizeof(kShapes[0]) == 12, "kShapes lists the shapes dispatched above");
+    static_assert(sizeof(kShapes) / sizeof(kShapes[0]) == 14, "kShapes lists the shapes dispatched above");
 }
 
 }  // namespace
@@ -824,7 +813,7 @@ bool launch_decode(const DecodeParams &params, bool fused, hipStream_t stream) {
     p.layer_bytes = p.g.n_groups * p.g.group_stride;
     p.div_qkv = make_fastdiv((uint32_t) p.q_per_kv);
     p.div_ctx = make_fastdiv((uint32_t) p.g.n_ctx);
-    const Shape s = pick_shape(units, p.n_layers, p.g.n_groups, p.q_per_kv, fused);
+    const Shape s = pick_shape(units, p.n_layers, p.g.n_groups, p.q_per_kv, fused, std::getenv("BMO_ATTN_SHAPE"));
     if (p.g.head_dim == 128)
         launch_shape<128>(p, fused, stream, s);
     else if (p.g.head_dim == 64)

@@ -1,8 +1,9 @@
 // decode_shape.hpp -- which workgroup shape a decode call takes (decode.hip).
-// Plain constexpr C++, so that a host test can walk the rule.
+// Plain C++, so that a host test can walk the rule.
 #pragma once
 
 #include <stdint.h>
+#include <stdio.h>
 
 #include <initializer_list>
 
@@ -13,9 +14,10 @@ struct Shape {
     int nw, pf, r;
 };
 
-// The shapes launch_shape instantiates.
-constexpr Shape kShapes[] = {{1, 1, 1}, {1, 2, 1}, {2, 1, 1}, {2, 2, 1}, {4, 1, 1}, {4, 2, 1}, {8, 1, 1}, {8, 2, 1},
-                             {1, 2, 2}, {2, 2, 2}, {4, 2, 2}, {1, 2, 4}};
+// The shapes launch_shape instantiates ({1, 3, 1}, {2, 1, 1} and {16, 1, 1}
+// only for BMO_ATTN_SHAPE).
+constexpr Shape kShapes[] = {{1, 1, 1}, {1, 2, 1}, {1, 3, 1}, {2, 1, 1},  {2, 2, 1}, {4, 1, 1}, {4, 2, 1},
+                             {8, 1, 1}, {8, 2, 1}, {16, 1, 1}, {1, 2, 2}, {2, 2, 2}, {4, 2, 2}, {1, 2, 4}};
 
 constexpr bool shape_instantiated(Shape s) {
     for (const Shape &k : kShapes)
@@ -101,5 +103,19 @@ constexpr bool default_shapes_instantiated() {
     return true;
 }
 static_assert(default_shapes_instantiated(), "every default decode shape has a kernel");
+
+// forced = "nw,pf[,r]" (the environment's BMO_ATTN_SHAPE, for tuning; null:
+// none) overrides the default; a shape without a kernel, or with an r that
+// does not divide the query heads of a kv head, falls back to one wave with
+// one group in flight.
+inline Shape pick_shape(int64_t units, int n_layers, int n_groups, int q_per_kv, bool fused, const char *forced) {
+    Shape s = default_shape(units, n_layers, n_groups, q_per_kv, fused);
+    if (forced) {
+        Shape o{0, 0, 1};
+        if (sscanf(forced, "%d,%d,%d", &o.nw, &o.pf, &o.r) >= 2) s = o;
+    }
+    if (!shape_instantiated(s) || q_per_kv % s.r != 0) s = Shape{1, 1, 1};
+    return s;
+}
 
 }  // namespace bmo

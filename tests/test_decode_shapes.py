@@ -1,5 +1,25 @@
 """The rule that gives a decode call its workgroup shape, on the host."""
+import pytest
+
+import test_gpu_decode_shapes
+import test_gpu_parity
 from _shapes import decode_shapes
+
+FORCED = sorted(set(test_gpu_parity.SHAPES) | set(test_gpu_decode_shapes.SHAPES))
+
+
+@pytest.mark.parametrize("forced", FORCED)
+def test_a_forced_shape_is_the_shape(forced):
+    """The shapes that the GPU tests force are compiled, so that none of those
+    tests runs the fallback in their place."""
+    want = (tuple(map(int, forced.split(","))) + (1,))[:3]
+    (got,) = decode_shapes([(24, 1, 32, 2 * want[2], True)], forced)
+    assert got[:3] == want
+
+
+def test_a_shape_without_a_kernel_falls_back():
+    for forced, per in (("3,1", 1), ("1,2,4", 2), ("1,2,0", 1), ("16,2", 1)):
+        assert decode_shapes([(24, 1, 32, per, True)], forced)[0][:3] == (1, 1, 1)
 
 
 def test_no_launch_of_too_many_threads():

@@ -10,6 +10,8 @@ from _ringsim import Mirror, check_close
 
 pytestmark = pytest.mark.gpu
 
+SHAPES = ["2,1", "2,2", "4,2", "8,2", "1,2,2", "2,2,2", "4,2,2"]
+
 
 def _check(gpu, n_batch, heads, kv, d, n_ctx, positions, fused, what):
     m = Mirror(gpu, 1, n_batch, kv, d, n_ctx)
@@ -59,7 +61,7 @@ def test_grouped_queries(gpu, heads, kv, d, n_ctx, n_batch, fused):
 
 
 @pytest.mark.parametrize("fused", [False, True])
-@pytest.mark.parametrize("shape", ["2,1", "2,2", "4,2", "8,2", "1,2,2", "2,2,2", "4,2,2"])
+@pytest.mark.parametrize("shape", SHAPES)
 @pytest.mark.parametrize("d,n_ctx,pos", [(128, 512, 700), (128, 512, 20), (128, 3000, 3100), (64, 8, 5),
                                          (128, 100, 95), (64, 200, 450)])
 def test_forced_shapes(gpu, monkeypatch, shape, d, n_ctx, pos, fused):

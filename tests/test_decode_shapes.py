@@ -5,7 +5,7 @@ import test_gpu_decode_shapes
 import test_gpu_parity
 from _shapes import decode_shapes
 
-FORCED = sorted(set(test_gpu_parity.SHAPES) | set(test_gpu_decode_shapes.SHAPES))
+FORCED = sorted(set(test_gpu_parity.SHAPES) | set(test_gpu_decode_shapes.SHAPES) | {"1,2,4"})
 
 
 @pytest.mark.parametrize("forced", FORCED)
@@ -30,3 +30,29 @@ def test_no_launch_of_too_many_threads():
              for per in (1, 2, 3, 4, 6, 16) for fused in (False, True)]
     for call, (nw, _, r, threads) in zip(calls, decode_shapes(calls)):
         assert threads == call[0] * 64 * nw < 2**32 and call[3] % r == 0, (call, nw, r)
+
+
+@pytest.mark.parametrize("fused,groups,per,low,low_shape,high_shape", [
+    (True, 32, 1, 127, (8, 1, 1), (4, 2, 1)), (False, 32, 1, 127, (8, 2, 1), (4, 2, 1)),
+    (True, 64, 1, 256, (8, 2, 1), (4, 2, 1)), (False, 64, 2, 256, (8, 2, 1), (4, 2, 2)),
+    (True, 32, 3, 768, (4, 2, 1), (2, 2, 1)), (False, 32, 3, 768, (4, 2, 1), (1, 2, 1)),
+    (True, 64, 1, 1536, (2, 2, 1), (1, 2, 1)), (False, 32, 1, 2048, (1, 2, 1), (4, 2, 1)),
+    (True, 32, 2, 512, (4, 2, 2), (2, 2, 2)), (False, 32, 4, 1536, (2, 2, 2), (1, 2, 4)),
+    (True, 31, 2, 1536, (2, 2, 2), (1, 2, 2)),
+])
+def test_lines_of_units(fused, groups, per, low, low_shape, high_shape):
+    got = decode_shapes([(low, 1, groups, per, fused), (low + 1, 1, groups, per, fused)])
+    assert [g[:3] for g in got] == [low_shape, high_shape]
+
+
+@pytest.mark.parametrize("groups", [1, 2, 7, 8, 32, 63, 64, 188])
+def test_a_launch_of_several_layers_splits_as_one(groups):
+    """The same waves a unit, and for fewer than eight the same groups in flight
+    (they decide how often V's code offset is settled)."""
+    calls = [(u, layers, groups, per, True) for u in (16, 32, 127, 128, 300, 1000) for per in (1, 2, 4)
+             for layers in (1, 2, 32)]
+    got = decode_shapes(calls)
+    for i in range(0, len(calls), 3):
+        for other in got[i + 1:i + 3]:
+            assert (other[0], other[2]) == (got[i][0], got[i][2])
+            assert other[1] == got[i][1] or got[i][0] == 8

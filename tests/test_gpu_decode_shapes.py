@@ -1,12 +1,13 @@
 """Waves per unit and groups in flight of the decode kernel against the float64
-oracle (|gpu - ref| <= 2e-3 + 1e-3 |ref|): the default rule on both sides of
-each of its lines, and the shapes that it chooses, forced, at runs of no, one
+oracle (|gpu - ref| <= 2e-3 + 1e-3 |ref|): the default rule near both sides of
+each of its lines (tests/test_decode_shapes.py has the lines themselves), and the shapes that it chooses, forced, at runs of no, one
 and few groups per wave."""
 import numpy as np
 import pytest
 
 import oracle
 from _ringsim import Mirror, check_close
+from _shapes import decode_shapes
 
 pytestmark = pytest.mark.gpu
 
@@ -34,19 +35,38 @@ def _check(gpu, n_batch, heads, kv, d, n_ctx, positions, fused, what):
         m.assert_ring_equal(0, s)
 
 
+# (entries, heads, slots), one kv head, head_dim 64 (32 slots a group): the shapes
+# (waves per unit, groups in flight, heads per workgroup) of the plain and the
+# fused call.  Neighbouring rows are the two sides of a line.
+DEFAULT = [
+    # heads odd: one head a workgroup
+    (1, 127, 288, (8, 2, 1), (8, 1, 1)), (3, 43, 288, (4, 2, 1), (4, 2, 1)),         # 127 | 129 units
+    (5, 51, 2048, (8, 2, 1), (8, 2, 1)), (1, 257, 2048, (4, 2, 1), (4, 2, 1)),       # 255 | 257 of 64 groups
+    (5, 51, 2016, (4, 2, 1), (4, 2, 1)),                                             # ... 63 groups
+    (3, 3, 2016, (8, 2, 1), (8, 1, 1)), (3, 3, 2048, (8, 2, 1), (8, 2, 1)),          # 63 | 64 groups, few units
+    (13, 59, 288, (4, 2, 1), (4, 2, 1)), (1, 769, 288, (1, 2, 1), (2, 2, 1)),        # 767 | 769
+    (5, 307, 288, (1, 2, 1), (2, 2, 1)), (29, 53, 288, (1, 2, 1), (1, 2, 1)),        # 1535 | 1537
+    (3, 341, 2048, (1, 2, 1), (2, 2, 1)), (3, 341, 2080, (1, 2, 1), (1, 2, 1)),      # 64 | 65 groups, 1023 units
+    (2, 1023, 1024, (1, 2, 1), (1, 2, 1)), (3, 683, 1024, (4, 2, 1), (1, 2, 1)),     # 2046 | 2049 of 32 groups
+    (3, 683, 992, (1, 2, 1), (1, 2, 1)),                                             # ... 31 groups
+    # heads even: grouped
+    (4, 64, 288, (4, 2, 1), (4, 2, 1)), (3, 86, 288, (4, 2, 2), (4, 2, 2)),          # 256 | 258 units
+    (4, 128, 288, (4, 2, 2), (4, 2, 2)), (2, 258, 288, (2, 2, 2), (2, 2, 2)),        # 512 | 516
+    (3, 512, 288, (2, 2, 2), (2, 2, 2)), (4, 388, 288, (1, 2, 4), (1, 2, 4)),        # 1536 | 1552, four heads
+    (4, 386, 992, (1, 2, 2), (1, 2, 2)), (4, 386, 1024, (2, 2, 2), (2, 2, 2)),       # 31 | 32 groups, two heads
+    (4, 128, 32, (1, 1, 1), (2, 1, 1)), (4, 128, 64, (2, 2, 2), (2, 2, 2)),          # 1 | 2 groups
+]
+
+
 @pytest.mark.parametrize("fused", [False, True])
-@pytest.mark.parametrize("n_batch,heads,n_ctx", [
-    (127, 1, 40), (2, 64, 40), (2, 128, 40), (257, 1, 40), (3, 256, 40), (769, 1, 40),      # 127 | 128, 256 | 257, 768 | 769
-    (3, 512, 40), (1537, 1, 33), (8, 256, 40), (683, 3, 40),     # 1536 | 1537, 2048 | 2049 units
-    (4, 512, 1024), (9, 228, 1024),                              # 2048 | 2052 units of 32 groups
-    (2, 4, 2016), (2, 4, 2048), (2, 80, 2016), (2, 80, 2048),    # 63 | 64 groups, few units
-    (2, 512, 2048), (2, 512, 2080),                              # 64 | 65 groups, 1024 units
-])
-def test_default_shapes(gpu, n_batch, heads, n_ctx, fused):
-    """One kv head, head_dim 64 (32 slots a group), entries with full and
-    partly filled windows."""
-    pos = [(n_ctx + 5 * s) if s % 3 else (7 * s) % n_ctx for s in range(n_batch)]
-    _check(gpu, n_batch, heads, 1, 64, n_ctx, pos, fused, f"{n_batch * heads} units, {n_ctx} slots")
+@pytest.mark.parametrize("n_batch,heads,n_ctx,plain_shape,fused_shape", DEFAULT)
+def test_default_shapes(gpu, n_batch, heads, n_ctx, plain_shape, fused_shape, fused):
+    """Entries with full and partly filled windows; the shape is the one named."""
+    units = n_batch * heads
+    (shape,) = decode_shapes([(units, 1, (n_ctx + 31) // 32, heads, fused)])
+    assert shape[:3] == (fused_shape if fused else plain_shape)
+    pos = [(n_ctx + 5 * s) if s % 3 != 1 else (7 * s) % n_ctx for s in range(n_batch)]
+    _check(gpu, n_batch, heads, 1, 64, n_ctx, pos, fused, f"{units} units, {n_ctx} slots")
 
 
 @pytest.mark.parametrize("fused", [False, True])
@@ -54,10 +74,16 @@ def test_default_shapes(gpu, n_batch, heads, n_ctx, fused):
 @pytest.mark.parametrize("d,n_ctx,n_batch", [(64, 40, 33), (128, 40, 70), (64, 8, 70), (128, 600, 200),
                                              (64, 500, 200)])
 def test_grouped_queries(gpu, heads, kv, d, n_ctx, n_batch, fused):
-    """2, 4, 8, 6 and 3 query heads a kv head on both sides of the grouped
-    shapes' lines (256, 512 and 1536 units, 32 groups)."""
+    """2, 4, 8, 6 and 3 query heads a kv head, both head dims, several kv heads."""
     pos = [(n_ctx + 5 * s) if s % 3 else (7 * s) % n_ctx for s in range(n_batch)]
     _check(gpu, n_batch, heads, kv, d, n_ctx, pos, fused, f"{heads}/{kv} heads, {n_batch} entries")
+
+
+@pytest.mark.parametrize("fused", [False, True])
+@pytest.mark.parametrize("d,n_ctx,pos", [(128, 512, 700), (128, 3000, 3100), (64, 8, 5), (64, 200, 450)])
+def test_forced_four_heads(gpu, monkeypatch, d, n_ctx, pos, fused):
+    monkeypatch.setenv("BMO_ATTN_SHAPE", "1,2,4")
+    _check(gpu, 2, 8, 2, d, n_ctx, [pos, max(0, pos - 19)], fused, "shape 1,2,4")
 
 
 @pytest.mark.parametrize("fused", [False, True])

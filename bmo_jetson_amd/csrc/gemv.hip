@@ -447,24 +447,44 @@ void launch_rows(const GemvParams &p, hipStream_t stream) {
                            stream, p);
 }
 
+// Two-row chunks per wave of 256 workgroups of 8.
+constexpr int stream_chunks_per_wave(int rows) {
+    return (int) (((int64_t) rows / 2 + rows % 2 + 256 * 8 - 1) / (256 * 8));
+}
+
+// Rows of at most 6144 columns whose byte length is a multiple of 16 (cols a
+// multiple of 256, so that every piece inside a chunk is loaded at its own
+// offset), in a 16-byte aligned matrix, take the streaming kernel
+// (BMO_GEMV_STREAM=0 turns it off, for comparison), on at most 256 workgroups
+// of 8 waves.  Chunks of up to 4608 bytes take 5 pieces, up to 6912 bytes 7
+// (56 KB of stages).  Past four chunks per wave only wide rows, whose chunks
+// are worth a load of their own round trip each.  us, streaming and
+// pair-walking kernel, weights from HBM (and from the last-level cache):
+//   17000 x 2048   7.56 /  7.37 (8.09 / 7.23)   32768 x 2048  11.3 / 11.0 (11.3 / 11.3)
+//   17000 x 2816   8.16 /  8.44 (8.64 / 8.13)   24576 x 2816  10.2 / 10.4 (10.1 / 10.4)
+//   17000 x 3328   8.47 /  8.89 (8.83 / 8.61)   24576 x 3328  10.2 / 11.0 (10.5 / 11.3)
+//   17000 x 3584   8.66 /  9.21 (9.00 / 9.21)   32768 x 3584  13.5 / 14.5 (13.6 / 14.5)
+//   17000 x 4096   9.02 /  9.84 (9.63 / 10.1)   32768 x 4096  14.7 / 15.8 (14.9 / 15.9)
+// and cached 22000 x 3072 10.1 / 10.5, 18500 x 3072 8.78 / 8.50.
+constexpr bool gemv_streams(int rows, int cols) {
+    const int npos = stream_chunks_per_wave(rows);
+    return cols <= 6144 && cols % 256 == 0 &&
+           (npos <= kStreamMaxPos || cols >= 3584 || (cols >= 3072 && npos > kStreamMaxPos + 1));
+}
+static_assert(gemv_streams(16384, 256) && gemv_streams(16385, 3584) && gemv_streams(20481, 3072) &&
+                  gemv_streams(2147483647, 6144),
+              "up to four chunks per wave, and past them wide rows");
+static_assert(!gemv_streams(16385, 3328) && !gemv_streams(20480, 3072) && !gemv_streams(32768, 2816) &&
+                  !gemv_streams(4096, 4224) && !gemv_streams(4096, 6400),
+              "narrow rows past four chunks per wave walk pairs");
+
 }  // namespace
 
 bool launch_gemv(const GemvParams &p, hipStream_t stream) {
-    // Rows of at most 6144 columns whose byte length is a multiple of 16
-    // (cols a multiple of 256, so that every piece inside a chunk is loaded
-    // at its own offset) and a 16-byte aligned matrix: the streaming kernel
-    // (BMO_GEMV_STREAM=0 turns it off, for comparison), on at most 256
-    // workgroups of 8 waves.  Chunks of up to 4608 bytes take 5 pieces, up to
-    // 6912 bytes 7 (56 KB of stages).  Past four chunks per wave only rows of
-    // 2048 columns or more: 32000 x 4096 14.6 us against the pair-walking
-    // kernel's 16.5, 30000 x 2048 11.1 / 11.3, but 30000 x 1536 10.75 / 10.6
-    // and 30000 x 1024 10.6 / 10.2, whose chunks are too short for a load of
-    // their own round trip each.
     const int n_chunks = p.rows / 2 + p.rows % 2;
-    const int npos = (int) (((int64_t) n_chunks + 256 * 8 - 1) / (256 * 8));
     const char *se = std::getenv("BMO_GEMV_STREAM");
-    if (p.cols <= 6144 && p.cols % 256 == 0 && (reinterpret_cast<uintptr_t>(p.w) & 15) == 0 &&
-        (npos <= kStreamMaxPos || p.cols >= 2048) && !(se && se[0] == '0')) {
+    if (gemv_streams(p.rows, p.cols) && (reinterpret_cast<uintptr_t>(p.w) & 15) == 0 && !(se && se[0] == '0')) {
+        const int npos = stream_chunks_per_wave(p.rows);
         if (p.cols <= 4096)
             launch_stream<5, 1>(p, npos, n_chunks, stream);
         else

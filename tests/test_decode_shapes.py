@@ -39,10 +39,22 @@ def test_no_launch_of_too_many_threads():
     (True, 64, 1, 1536, (2, 2, 1), (1, 2, 1)), (False, 32, 1, 2048, (1, 2, 1), (4, 2, 1)),
     (True, 32, 2, 512, (4, 2, 2), (2, 2, 2)), (False, 32, 4, 1536, (2, 2, 2), (1, 2, 4)),
     (True, 31, 2, 1536, (2, 2, 2), (1, 2, 2)),
+    (True, 1, 1, 256, (2, 1, 1), (1, 1, 1)), (True, 3, 1, 511, (2, 1, 1), (1, 2, 1)),
+    (False, 6, 1, 512, (4, 2, 1), (2, 2, 1)), (True, 2, 4, 512, (2, 2, 2), (1, 2, 1)),
 ])
 def test_lines_of_units(fused, groups, per, low, low_shape, high_shape):
     got = decode_shapes([(low, 1, groups, per, fused), (low + 1, 1, groups, per, fused)])
     assert [g[:3] for g in got] == [low_shape, high_shape]
+
+
+@pytest.mark.parametrize("fused,waves", [
+    # 1, 2, ... groups: no more waves on short windows than pay there
+    (True, [1, 1, 1, 2, 1, 2, 2, 1, 2, 2, 1, 2, 2, 4, 4]),
+    (False, [1, 1, 2, 2, 1, 2, 2, 1, 2, 2, 2, 2, 2, 2, 2])])
+@pytest.mark.parametrize("units", [513, 640, 768])
+def test_waves_of_short_windows(units, fused, waves):
+    got = decode_shapes([(units, 1, n + 1, 1, fused) for n in range(len(waves))])
+    assert [g[0] for g in got] == waves
 
 
 @pytest.mark.parametrize("groups", [1, 2, 7, 8, 32, 63, 64, 188])

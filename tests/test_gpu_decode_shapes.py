@@ -44,17 +44,27 @@ DEFAULT = [
     (5, 51, 2048, (8, 2, 1), (8, 2, 1)), (1, 257, 2048, (4, 2, 1), (4, 2, 1)),       # 255 | 257 of 64 groups
     (5, 51, 2016, (4, 2, 1), (4, 2, 1)),                                             # ... 63 groups
     (3, 3, 2016, (8, 2, 1), (8, 1, 1)), (3, 3, 2048, (8, 2, 1), (8, 2, 1)),          # 63 | 64 groups, few units
-    (13, 59, 288, (4, 2, 1), (4, 2, 1)), (1, 769, 288, (1, 2, 1), (2, 2, 1)),        # 767 | 769
+    (13, 59, 288, (2, 2, 1), (2, 2, 1)), (1, 769, 288, (1, 2, 1), (2, 2, 1)),        # 767 | 769
     (5, 307, 288, (1, 2, 1), (2, 2, 1)), (29, 53, 288, (1, 2, 1), (1, 2, 1)),        # 1535 | 1537
     (3, 341, 2048, (1, 2, 1), (2, 2, 1)), (3, 341, 2080, (1, 2, 1), (1, 2, 1)),      # 64 | 65 groups, 1023 units
     (2, 1023, 1024, (1, 2, 1), (1, 2, 1)), (3, 683, 1024, (4, 2, 1), (1, 2, 1)),     # 2046 | 2049 of 32 groups
     (3, 683, 992, (1, 2, 1), (1, 2, 1)),                                             # ... 31 groups
+    (1, 255, 32, (1, 1, 1), (2, 1, 1)), (1, 257, 32, (1, 1, 1), (1, 1, 1)),          # 255 | 257 of 1 group
+    (1, 127, 64, (2, 1, 1), (2, 1, 1)),                                              # fewer groups than waves
+    (7, 73, 96, (2, 1, 1), (2, 1, 1)), (512, 1, 96, (2, 1, 1), (1, 2, 1)),           # 511 | 512 of 3 groups
+    (512, 1, 128, (4, 1, 1), (4, 2, 1)), (3, 171, 96, (2, 2, 1), (1, 2, 1)),         # 512 of 4 | 513 of 3
+    (3, 171, 256, (1, 2, 1), (1, 2, 1)), (3, 171, 288, (2, 2, 1), (2, 2, 1)),        # 513 units, 8 | 9 groups
+    (3, 171, 352, (2, 2, 1), (1, 2, 1)),                                             # ... 11
+    (3, 171, 416, (2, 2, 1), (2, 2, 1)), (3, 171, 448, (2, 2, 1), (4, 2, 1)),        # ... 13 | 14
+    (3, 171, 992, (2, 2, 1), (4, 2, 1)), (3, 171, 1024, (4, 2, 1), (4, 2, 1)),       # ... 31 | 32
+    (3, 341, 64, (1, 2, 1), (1, 2, 1)), (3, 341, 96, (1, 2, 1), (2, 2, 1)),          # 2 | 3 groups, 1023 units
     # heads even: grouped
     (4, 64, 288, (4, 2, 1), (4, 2, 1)), (3, 86, 288, (4, 2, 2), (4, 2, 2)),          # 256 | 258 units
     (4, 128, 288, (4, 2, 2), (4, 2, 2)), (2, 258, 288, (2, 2, 2), (2, 2, 2)),        # 512 | 516
     (3, 512, 288, (2, 2, 2), (2, 2, 2)), (4, 388, 288, (1, 2, 4), (1, 2, 4)),        # 1536 | 1552, four heads
     (4, 386, 992, (1, 2, 2), (1, 2, 2)), (4, 386, 1024, (2, 2, 2), (2, 2, 2)),       # 31 | 32 groups, two heads
-    (4, 128, 32, (1, 1, 1), (2, 1, 1)), (4, 128, 64, (2, 2, 2), (2, 2, 2)),          # 1 | 2 groups
+    (4, 128, 32, (1, 1, 1), (1, 1, 1)), (4, 128, 64, (2, 2, 2), (2, 2, 2)),          # 1 | 2 groups
+    (3, 172, 64, (1, 2, 1), (1, 2, 1)), (4, 388, 64, (1, 2, 4), (1, 2, 4)),          # 2 groups, 516 | 1552
 ]
 
 

@@ -50,6 +50,7 @@
 #include <math.h>
 
 #include "kernels.hpp"
+#include "prefill_shape.hpp"
 #include "q4_0_device.hpp"
 
 namespace bmo {
@@ -226,16 +227,6 @@ __global__ __launch_bounds__(256) void commit_kernel(PrefillParams p) {
         *reinterpret_cast<const uint32_t *>(src + p.sg.scale_offset(i, blk));
 }
 
-// Launch bounds: four waves per SIMD, one workgroup of 16 waves per CU or two
-// of 8, at most 128 VGPRs each, which holds the accumulators, the query
-// operands and the fetched tile bytes without spilling.
-//
-// DIRECT: every (entry, kv head) stripe is read by this one workgroup (one
-// query head per kv head, the whole chunk in one workgroup).  The workgroup
-// then quantizes its chunk's K/V itself into LDS (the staging stripe's role),
-// reads the chunk's keys from there, and writes the chunk's blocks into the
-// ring during the tile loop, each once no wave reads its slot's old contents
-// from memory any more; no stage or commit kernel runs.
 // Phase timestamps, in a diagnostic build only (BMO_PREFILL_PHASES=1,
 // libbmo_attn_phases.so, which bench.py --prefill-phases reads): lane 0 of
 // every wave of the first 512 workgroups records s_memtime at its phase
@@ -278,6 +269,16 @@ __device__ uint64_t g_prefill_phases[kPhaseUnits * 16 * kPhaseRec];
     } while (0)
 #endif
 
+// Launch bounds: four waves per SIMD, one workgroup of 16 waves per CU or two
+// of 8, at most 128 VGPRs each, which holds the accumulators, the query
+// operands and the fetched tile bytes without spilling.
+//
+// DIRECT: every (entry, kv head) stripe is read by this one workgroup (one
+// query head per kv head, the whole chunk in one workgroup).  The workgroup
+// then quantizes its chunk's K/V itself into LDS (the staging stripe's role),
+// reads the chunk's keys from there, and writes the chunk's blocks into the
+// ring during the tile loop, each once no wave reads its slot's old contents
+// from memory any more; no stage or commit kernel runs.
 template <int D, int QW, int QB, int KS, bool DIRECT, bool ALIGNED>
 __global__ __launch_bounds__(64 * QW, 4) void prefill_kernel(PrefillParams p) {
     static_assert(!DIRECT || ALIGNED, "the direct path serves rings of a multiple of 32 slots");
@@ -571,7 +572,6 @@ __global__ __launch_bounds__(64 * QW, 4) void prefill_kernel(PrefillParams p) {
             }
         }
     };
-
 
     // Loads, in the order they are waited for (loads return in order): the
     // query rows, the first PF tiles, then (DIRECT) the chunk's bf16 K/V; the
@@ -1001,7 +1001,8 @@ __global__ __launch_bounds__(64 * QW, 4) void prefill_kernel(PrefillParams p) {
 
     // KS: the waves of a query block each hold the softmax state of half the
     // tiles.  The second hands its sums over in the tile buffers (nobody reads
-    // a tile any more), with each query's offset and weight sum, and the first joins them at the larger offset and stores.
+    // a tile any more), with each query's offset and weight sum, and the first
+    // joins them at the larger offset and stores.
     if constexpr (KS > 1) {
         constexpr int XQ = (NT / 2) * 64;  // float4s of half a wave's sums
         static_assert(QB == 1 && sizeof(sV) >= QW / KS * XQ * sizeof(float4_t) &&
@@ -1100,72 +1101,9 @@ namespace {
 // 106.5-106.6 us (ring history full), 60.7 vs 69.1 us (empty).
 // Fewer queries a workgroup mean as many tiles to dequantize for less work,
 // so smaller ones pay where 256-query workgroups leave CUs idle: few units,
-// short chunks, a nearly empty last round (below).
+// short chunks, a nearly empty last round (prefill_shape.hpp).
 constexpr int kQW = 16;
-constexpr int kQB = 1;
 constexpr int kQT = 16 * kQB * kQW;  // queries per workgroup of the direct path
-
-// Workgroup of the staged path: qw waves, ks of them on each block of 16
-// queries.
-struct StagedShape {
-    int qw, ks;
-    constexpr int queries() const { return 16 * kQB * qw / ks; }
-};
-constexpr StagedShape kStagedShapes[] = {{16, 1}, {16, 2}, {8, 1}, {8, 2}};
-
-// The time of a staged call's workgroups in units of one round of 256
-// workgroups of 16 waves x 16 queries, one a CU.  A 16-wave workgroup fills a
-// CU; two 8-wave ones fit, and slow each other down.  Measured with 8 of 32
-// heads' K/V, 1024 slots, 500 and 256 tokens (us; 16 x 1, 16 x 2, 8 x 1, 8 x
-// 2): 1 session 61.7 / 50.2 / 54.9 / 43.8, 2 sessions 62.9 / 51.0 / 56.1 /
-// 59.6, 3 sessions 64.7 / 92.8 / 76.7 / 87.1, 16 x 256 tokens 124 / 178 / 140
-// / 196; 24 sessions x 64 tokens 120.9 / 118.5 / 87.7 / 85.8.
-constexpr double staged_cost(const StagedShape &s, int64_t workgroups) {
-    const int per_cu = s.qw == 16 ? 1 : 2;
-    const double alone = s.qw == 16 ? (s.ks == 1 ? 1.0 : 0.81) : (s.ks == 1 ? 0.88 : 0.71);
-    const double shared = s.ks == 1 ? 1.155 : 0.95;
-    const int64_t round = 256 * per_cu;
-    const int64_t rest = workgroups % round;
-    return (double) (workgroups / round) * (per_cu == 1 ? alone : shared) +
-           (rest == 0 ? 0.0 : rest <= 256 ? alone : shared);
-}
-
-// The cheapest shape; a smaller one only if it saves a twentieth.
-constexpr StagedShape staged_shape(int64_t units, int n_tok) {
-    StagedShape best = kStagedShapes[0];
-    double cost = 0.95 * staged_cost(best, units * ((n_tok + best.queries() - 1) / best.queries()));
-    for (int i = 1; i < 4; ++i) {
-        const StagedShape s = kStagedShapes[i];
-        const double c = staged_cost(s, units * ((n_tok + s.queries() - 1) / s.queries()));
-        if (c < cost) {
-            best = s;
-            cost = c;
-        }
-    }
-    return best;
-}
-// The units that go ahead in full rounds of the first shape, when the rest in
-// a shape of its own then takes a twentieth less in all than every unit in
-// one (0: one launch).  A second launch costs as much as about 0.05 rounds.
-// 160 units of 500 tokens, 320 workgroups of 256 queries: 128 units in one
-// round and 32 in 256 workgroups of 64 queries, XX us against 110.
-constexpr int64_t staged_full_units(int64_t units, int n_tok) {
-    auto cost = [=](int64_t n) {
-        const StagedShape s = staged_shape(n, n_tok);
-        return staged_cost(s, n * ((n_tok + s.queries() - 1) / s.queries()));
-    };
-    const int64_t n_qt = (n_tok + kStagedShapes[0].queries() - 1) / kStagedShapes[0].queries();
-    const int64_t rounds = units * n_qt / 256;
-    const int64_t full = rounds * 256 / n_qt;
-    if (full == 0 || full == units) return 0;
-    return (double) rounds + 0.05 + cost(units - full) < 0.95 * cost(units) ? full : 0;
-}
-static_assert(staged_full_units(160, 500) == 128 && staged_full_units(512, 256) == 0,
-              "a quarter of a round goes apart, full rounds do not");
-
-static_assert(staged_shape(512, 256).qw == 16 && staged_shape(512, 256).ks == 1, "full rounds: 256 queries");
-static_assert(staged_shape(32, 500).qw == 8 && staged_shape(32, 500).ks == 2, "256 workgroups of 64 queries");
-static_assert(staged_shape(64, 500).qw == 16 && staged_shape(64, 500).ks == 2, "256 workgroups of 128 queries");
 
 template <int D, int QW, int KS, bool DIRECT>
 void launch_attention(const PrefillParams &p, int64_t units, hipStream_t stream) {

@@ -1,18 +1,31 @@
-"""Test helper: the decode calls' workgroup shapes, from the rule that the
-library is compiled with (bmo_jetson_amd/csrc/decode_shape.hpp)."""
+"""Test helper: the workgroup shapes of decode and staged prefill calls, from the
+rules that the library is compiled with (bmo_jetson_amd/csrc/decode_shape.hpp
+and prefill_shape.hpp)."""
 import os
 import subprocess
 
-EXE = os.path.join(os.path.dirname(os.path.abspath(__file__)), "build", "decode_shape_check")
+BUILD = os.path.join(os.path.dirname(os.path.abspath(__file__)), "build")
+
+
+def _ask(program, lines):
+    exe = os.path.join(BUILD, program)
+    assert os.path.exists(exe), f"tests/build/{program} is not built (run __graft_entry__.build())"
+    res = subprocess.run([exe], input="".join(l + "\n" for l in lines), capture_output=True, text=True,
+                         timeout=60, check=True)
+    out = [tuple(map(int, line.split())) for line in res.stdout.splitlines()]
+    assert len(out) == len(lines)
+    return out
 
 
 def decode_shapes(calls, forced="-"):
     """(waves per unit, groups in flight, heads per workgroup, threads) of each
     (units, layers, groups, query heads per kv head, fused), with the shape
     that BMO_ATTN_SHAPE forces."""
-    assert os.path.exists(EXE), "tests/build/decode_shape_check is not built (run __graft_entry__.build())"
-    text = "".join("%d %d %d %d %d %s\n" % (u, layers, n, per, bool(f), forced) for u, layers, n, per, f in calls)
-    res = subprocess.run([EXE], input=text, capture_output=True, text=True, timeout=60, check=True)
-    out = [tuple(map(int, line.split())) for line in res.stdout.splitlines()]
-    assert len(out) == len(calls)
-    return out
+    return _ask("decode_shape_check",
+                ["%d %d %d %d %d %s" % (u, layers, n, per, bool(f), forced) for u, layers, n, per, f in calls])
+
+
+def staged_shapes(calls):
+    """(units in full rounds of 16 waves x 16 queries, waves per workgroup and
+    per block of queries of the rest) of each (units, tokens)."""
+    return _ask("prefill_shape_check", ["%d %d" % c for c in calls])

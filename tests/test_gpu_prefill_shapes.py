@@ -1,6 +1,6 @@
 """Staged prefill in each of its workgroup shapes against the float64 oracle
 (|gpu - ref| <= 2e-3 + 1e-3 |ref|): 16 or 8 waves, one or two on each block
-of 16 queries, picked by the number of units and the chunk's length, at chunks
+of 16 queries, picked by the number of units and the chunk's length (asserted), at chunks
 around a workgroup's queries, rings on and off the 32-slot grid, and queries
 that see keys in only one half of the tiles.  The committed ring is exact."""
 import numpy as np
@@ -8,24 +8,37 @@ import pytest
 
 import oracle
 from _ringsim import Mirror, check_close
+from _shapes import staged_shapes
 
 pytestmark = pytest.mark.gpu
 
 
+# entries, heads, kv heads, slots, position, tokens, and the shape: units in full
+# rounds of 16 waves x 16 queries, waves per workgroup and per block of queries
+# of the rest
+STAGED = [
+    (1, 4, 2, 128, 200, 63, (0, 8, 2)), (1, 4, 2, 128, 200, 65, (0, 8, 2)),  # 64-query workgroups, an edge and past it
+    (1, 4, 2, 96, 0, 1, (0, 8, 2)),                # one key: the second wave of a block sees none
+    (1, 4, 2, 100, 40, 33, (0, 8, 2)),             # off the 32-slot grid
+    (1, 2, 2, 300, 500, 300, (0, 8, 2)),           # more than 256 tokens, one head a kv head
+    (3, 32, 2, 96, 130, 90, (0, 8, 2)),            # 96 units
+    (9, 32, 1, 40, 70, 33, (0, 8, 2)),             # 288 units: past one round of lone workgroups
+    (8, 32, 4, 64, 90, 17, (0, 8, 2)),             # 256 units
+    (20, 32, 1, 40, 50, 20, (0, 8, 2)),            # 640 units: past a round of two workgroups a CU
+    (4, 32, 2, 160, 200, 129, (0, 16, 2)),         # 128-query workgroups, an edge and past it
+    (3, 32, 2, 300, 280, 200, (0, 16, 2)),         # off the grid
+    (3, 32, 2, 256, 0, 256, (0, 16, 2)),           # empty history: half the tiles at most
+    (16, 32, 1, 96, 70, 70, (0, 8, 1)),            # 8 waves, 128 queries
+    (16, 32, 1, 160, 100, 128, (0, 8, 1)), (9, 32, 2, 100, 130, 100, (0, 8, 1)),
+    (5, 32, 2, 160, 100, 130, (0, 16, 1)),         # 160 units, 130 tokens
+    (5, 32, 2, 512, 100, 500, (128, 8, 2)),        # 128 units in a full round, 32 apart
+]
+
+
 @pytest.mark.parametrize("d", [64, 128])
-@pytest.mark.parametrize("n_batch,heads,kv,n_ctx,pos0,n_tok", [
-    (1, 4, 2, 128, 200, 63), (1, 4, 2, 128, 200, 65),     # 64-query workgroups, an edge and past it
-    (1, 4, 2, 96, 0, 1),                                  # one key: the second wave of a block sees none
-    (1, 4, 2, 100, 40, 33),                               # off the 32-slot grid
-    (1, 2, 2, 300, 500, 300),                             # more than 256 tokens, one head a kv head
-    (3, 32, 2, 96, 130, 90),                              # 96 units
-    (9, 32, 1, 40, 70, 33),                               # 288 units of one workgroup: 8 waves, 128 queries
-    (5, 32, 2, 160, 100, 130),                            # 160 units, 130 tokens
-    (8, 32, 4, 64, 90, 17),                               # 256 units
-    (20, 32, 1, 40, 50, 20),                              # 640 units
-    (5, 32, 2, 512, 100, 500),                            # 128 units in a full round, 32 apart
-])
-def test_staged_shapes(gpu, d, n_batch, heads, kv, n_ctx, pos0, n_tok):
+@pytest.mark.parametrize("n_batch,heads,kv,n_ctx,pos0,n_tok,shape", STAGED)
+def test_staged_shapes(gpu, d, n_batch, heads, kv, n_ctx, pos0, n_tok, shape):
+    assert staged_shapes([(n_batch * heads, n_tok)]) == [shape]
     m = Mirror(gpu, 1, n_batch, kv, d, n_ctx)
     pos = [max(0, pos0 - 7 * (b % 3)) for b in range(n_batch)]
     for b in range(n_batch):

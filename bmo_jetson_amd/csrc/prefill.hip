@@ -382,7 +382,8 @@ __global__ __launch_bounds__(64 * QW, 4) void prefill_kernel(PrefillParams p) {
     const int n_tiles = n_rt + (p_last - c_start) / kTK + 1;
     // (helpers capture by value: a select between captured references can
     // keep the closures in scratch memory, as noted at src_diff below)
-    auto tile_t0 = [=](int T) { return T < n_rt ? r_start + T * kTK : c_start + (T - n_rt) * kTK; };
+    const int c_base = c_start - n_rt * kTK;
+    auto tile_t0 = [=](int T) { return T * kTK + (T < n_rt ? r_start : c_base); };
     // Processing order.  A query at position P sees ring tile r only while
     // P <= (last key of r) + n_ctx - 1, and chunk tile c only from P >=
     // (first key of c) on: ring tiles are seen by the early waves, chunk
@@ -398,13 +399,24 @@ __global__ __launch_bounds__(64 * QW, 4) void prefill_kernel(PrefillParams p) {
     // softmax is online.)
     const int gam = (r_start + kTK - 2 - p_first + n_ctx) / kTK + 1 + (p_first - c_start) / kTK;
     const int n_pair = max(0, min(n_rt, n_tiles - n_rt - gam));
-    // (selects, not branches: the callers' blocks stay whole)
+    // (selects, not branches: the callers' blocks stay whole.  gam >= 1, so an
+    // unpaired chunk tile from gam on follows every unpaired ring tile, and one
+    // select serves; with nested ones hipcc made branches, 16 more per four
+    // tiles of a wave that only multiplies, and long windows at head_dim 64
+    // took 2 to 3 % longer.  The direct kernel of head_dim 128 would spill a
+    // register that way.)
+    const int odd_off = n_rt + gam, skip_at = n_pair + odd_off;
     auto tile_of = [=](int i) {
-        const int paired = (i & 1) ? n_rt + (i >> 1) + gam : (i >> 1);
-        const int j = i - 2 * n_pair;             // position among the unpaired tiles
-        const int jc = j - (n_rt - n_pair);       // ... among the unpaired chunk tiles
-        const int rest = j < n_rt - n_pair ? n_pair + j : n_rt + (jc < gam ? jc : jc + n_pair);
-        return i < 2 * n_pair ? paired : rest;    // padding positions map to themselves
+        const int paired = (i >> 1) + (i & 1 ? odd_off : 0);
+        int rest;
+        if constexpr (DIRECT) {
+            const int j = i - 2 * n_pair;         // position among the unpaired tiles
+            const int jc = j - (n_rt - n_pair);   // ... among the unpaired chunk tiles
+            rest = j < n_rt - n_pair ? n_pair + j : n_rt + (jc < gam ? jc : jc + n_pair);
+        } else {
+            rest = i - (i < skip_at ? n_pair : 0);
+        }
+        return i < 2 * n_pair ? paired : rest;  // padding positions map to themselves
     };
     const uint8_t *ring = p.base + p.g.stripe_offset(p.layer, sid, kvh);
     const uint8_t *stage = p.stage + p.sg.stripe_offset(0, b, kvh);

@@ -1148,9 +1148,9 @@ template <int D>
 void launch_attention(const PrefillParams &p, bool direct, hipStream_t stream) {
     const int64_t units = (int64_t) p.n_batch * p.n_heads;
     if (direct) return launch_attention<D, kQW, 1, true>(p, units, stream);
-    const int64_t full = staged_full_units(units, p.n_tok);
+    const int64_t full = staged_full_units(units, p.n_tok, p.g.n_ctx);
     if (full > 0) launch_staged<D>(p, 0, full, kStagedShapes[0], stream);
-    if (full < units) launch_staged<D>(p, full, units - full, staged_shape(units - full, p.n_tok), stream);
+    if (full < units) launch_staged<D>(p, full, units - full, staged_shape(units - full, p.n_tok, p.g.n_ctx), stream);
 }
 
 }  // namespace

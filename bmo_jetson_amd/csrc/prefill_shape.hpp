@@ -23,13 +23,11 @@ constexpr StagedShape kStagedShapes[] = {{16, 1}, {16, 2}, {8, 1}, {8, 2}};
 // 2): 1 session 61.7 / 50.2 / 54.9 / 43.8, 2 sessions 62.9 / 51.0 / 56.1 /
 // 59.6, 3 sessions 64.7 / 92.8 / 76.7 / 87.1, 16 x 256 tokens 124 / 178 / 140
 // / 196; 24 sessions x 64 tokens 120.9 / 118.5 / 87.7 / 85.8.  The constants
-// stand for other rings and for head_dim 64 too: of 40 staged calls of 1 to
-// 24 sessions, 16 to 600 tokens, 64 to 3000 slots and both head dims, 38 take
-// no longer than in 16 x 1 (22.0 against 26.1 us for 16 tokens of one session
-// on 512 slots, 21.2 / 23.3 for 64 tokens at d64, 49.3 / 68.1 for 2 x 300
-// tokens, 2048 slots, d64, 165 / 237 for 3 x 600, 3000 slots), and two on
-// nearly empty rings at d64 a little (10 x 130 tokens 30.2 / 29.4, 6 x 128
-// 15.7 / 14.6), since the window does not enter.
+// stand for other rings and for head_dim 64 too, though the window does not
+// enter: of 576 calls of 1 to 24 sessions (8 of 32 heads' K/V), 16 to 400
+// tokens, 512 slots empty and full and 2048 full, both head dims, none takes
+// longer than with 16 x 1 throughout but 12 sessions x 256 tokens on an empty
+// ring at d64 (31.1 against 30.0 us; full 52 / 57).
 constexpr double staged_cost(const StagedShape &s, int64_t workgroups) {
     const int per_cu = s.qw == 16 ? 1 : 2;
     const double alone = s.qw == 16 ? (s.ks == 1 ? 1.0 : 0.81) : (s.ks == 1 ? 0.88 : 0.71);
@@ -40,12 +38,18 @@ constexpr double staged_cost(const StagedShape &s, int64_t workgroups) {
            (rest == 0 ? 0.0 : rest <= 256 ? alone : shared);
 }
 
-// The cheapest shape; a smaller one only if it saves a twentieth.
-constexpr StagedShape staged_shape(int64_t units, int n_tok) {
+// The cheapest shape; a smaller one only if it saves a twentieth.  Up to 128
+// tokens 16 x 2 has as many workgroups as 16 x 1 and twice the waves that load
+// queries, which only a long window repays: on rings of up to 512 slots 8 x 1
+// takes its place (6 sessions x 128 tokens, d128, us in 8 x 1, 16 x 2 and 16
+// x 1: 512 slots empty 17.0 / 19.8 / 17.4, full 34.7 / 35.2 / 35.3; 2048 slots
+// full 79.7 / 69.3 / 80.6).
+constexpr StagedShape staged_shape(int64_t units, int n_tok, int n_ctx) {
     StagedShape best = kStagedShapes[0];
     double cost = 0.95 * staged_cost(best, units * ((n_tok + best.queries() - 1) / best.queries()));
     for (int i = 1; i < 4; ++i) {
         const StagedShape s = kStagedShapes[i];
+        if (s.qw == 16 && n_tok <= s.queries() && n_ctx <= 512) continue;
         const double c = staged_cost(s, units * ((n_tok + s.queries() - 1) / s.queries()));
         if (c < cost) {
             best = s;
@@ -61,9 +65,9 @@ constexpr StagedShape staged_shape(int64_t units, int n_tok) {
 // 160 units of 500 tokens (8 of 32 heads' K/V, 1000 slots), 320 workgroups of
 // 256 queries: 128 units in one round and 32 in 256 workgroups of 64 queries,
 // 93.4 us a call against 104.9 in one launch.
-constexpr int64_t staged_full_units(int64_t units, int n_tok) {
+constexpr int64_t staged_full_units(int64_t units, int n_tok, int n_ctx) {
     auto cost = [=](int64_t n) {
-        const StagedShape s = staged_shape(n, n_tok);
+        const StagedShape s = staged_shape(n, n_tok, n_ctx);
         return staged_cost(s, n * ((n_tok + s.queries() - 1) / s.queries()));
     };
     const int64_t n_qt = (n_tok + kStagedShapes[0].queries() - 1) / kStagedShapes[0].queries();
@@ -72,10 +76,10 @@ constexpr int64_t staged_full_units(int64_t units, int n_tok) {
     if (full == 0 || full == units) return 0;
     return (double) rounds + 0.05 + cost(units - full) < 0.95 * cost(units) ? full : 0;
 }
-static_assert(staged_full_units(160, 500) == 128 && staged_full_units(512, 256) == 0,
+static_assert(staged_full_units(160, 500, 1000) == 128 && staged_full_units(512, 256, 512) == 0,
               "a quarter of a round goes apart, full rounds do not");
-static_assert(staged_shape(512, 256).qw == 16 && staged_shape(512, 256).ks == 1, "full rounds: 256 queries");
-static_assert(staged_shape(32, 500).qw == 8 && staged_shape(32, 500).ks == 2, "256 workgroups of 64 queries");
-static_assert(staged_shape(64, 500).qw == 16 && staged_shape(64, 500).ks == 2, "256 workgroups of 128 queries");
+static_assert(staged_shape(512, 256, 1024).qw == 16 && staged_shape(512, 256, 1024).ks == 1, "full rounds: 256 queries");
+static_assert(staged_shape(32, 500, 1024).qw == 8 && staged_shape(32, 500, 1024).ks == 2, "256 workgroups of 64 queries");
+static_assert(staged_shape(64, 500, 1024).qw == 16 && staged_shape(64, 500, 1024).ks == 2, "256 workgroups of 128 queries");
 
 }  // namespace bmo

@@ -27,5 +27,5 @@ def decode_shapes(calls, forced="-"):
 
 def staged_shapes(calls):
     """(units in full rounds of 16 waves x 16 queries, waves per workgroup and
-    per block of queries of the rest) of each (units, tokens)."""
-    return _ask("prefill_shape_check", ["%d %d" % c for c in calls])
+    per block of queries of the rest) of each (units, tokens, slots)."""
+    return _ask("prefill_shape_check", ["%d %d %d" % c for c in calls])

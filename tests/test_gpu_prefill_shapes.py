@@ -28,6 +28,7 @@ STAGED = [
     (4, 32, 2, 160, 200, 129, (0, 16, 2)),         # 128-query workgroups, an edge and past it
     (3, 32, 2, 300, 280, 200, (0, 16, 2)),         # off the grid
     (3, 32, 2, 256, 0, 256, (0, 16, 2)),           # empty history: half the tiles at most
+    (6, 32, 2, 544, 600, 100, (0, 16, 2)), (6, 32, 2, 512, 600, 100, (0, 8, 1)),  # past | up to 512 slots
     (16, 32, 1, 96, 70, 70, (0, 8, 1)),            # 8 waves, 128 queries
     (16, 32, 1, 160, 100, 128, (0, 8, 1)), (9, 32, 2, 100, 130, 100, (0, 8, 1)),
     (5, 32, 2, 160, 100, 130, (0, 16, 1)),         # 160 units, 130 tokens
@@ -38,7 +39,7 @@ STAGED = [
 @pytest.mark.parametrize("d", [64, 128])
 @pytest.mark.parametrize("n_batch,heads,kv,n_ctx,pos0,n_tok,shape", STAGED)
 def test_staged_shapes(gpu, d, n_batch, heads, kv, n_ctx, pos0, n_tok, shape):
-    assert staged_shapes([(n_batch * heads, n_tok)]) == [shape]
+    assert staged_shapes([(n_batch * heads, n_tok, n_ctx)]) == [shape]
     m = Mirror(gpu, 1, n_batch, kv, d, n_ctx)
     pos = [max(0, pos0 - 7 * (b % 3)) for b in range(n_batch)]
     for b in range(n_batch):

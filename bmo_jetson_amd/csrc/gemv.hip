@@ -335,7 +335,7 @@ __global__ __launch_bounds__(512) void gemv_stream_kernel(GemvParams p) {
     // that are read (rows are a multiple of 16 bytes), and a wave without
     // chunks reads the last chunk
     auto issue = [&](int k, u32x4_t (&w)[NPC]) {
-        const int64_t cbase = min((int64_t) c0 + (int64_t) k * stride, (int64_t) n_chunks - 1) * chunk_bytes;
+        const int64_t cbase = (int64_t) min(c0 + k * stride, n_chunks - 1) * chunk_bytes;
         const int64_t last = min(cbase + chunk_bytes, mat_bytes) - 16;
 #pragma unroll
         for (int j = 0; j < NPC; ++j)
@@ -398,10 +398,10 @@ __global__ __launch_bounds__(512) void gemv_stream_kernel(GemvParams p) {
         if (lane == 0) {
 #pragma unroll
             for (int k = 0; k < NPOS; ++k) {
-                const int64_t row = ((int64_t) c0 + (int64_t) (k0 + k) * stride) * R;
+                const uint32_t row = (uint32_t) (c0 + (k0 + k) * stride) * R;
 #pragma unroll
                 for (int r = 0; r < R; ++r)
-                    if (k0 + k < n_mine && row + r < p.rows) p.y[row + r] = yv[k][r];
+                    if (k0 + k < n_mine && row + r < (uint32_t) p.rows) p.y[row + r] = yv[k][r];
             }
         }
     }
@@ -459,13 +459,18 @@ constexpr int stream_chunks_per_wave(int rows) {
 // of 8 waves.  Chunks of up to 4608 bytes take 5 pieces, up to 6912 bytes 7
 // (56 KB of stages).  Past four chunks per wave only wide rows, whose chunks
 // are worth a load of their own round trip each.  us, streaming and
-// pair-walking kernel, weights from HBM (and from the last-level cache):
-//   17000 x 2048   7.56 /  7.37 (8.09 / 7.23)   32768 x 2048  11.3 / 11.0 (11.3 / 11.3)
-//   17000 x 2816   8.16 /  8.44 (8.64 / 8.13)   24576 x 2816  10.2 / 10.4 (10.1 / 10.4)
-//   17000 x 3328   8.47 /  8.89 (8.83 / 8.61)   24576 x 3328  10.2 / 11.0 (10.5 / 11.3)
-//   17000 x 3584   8.66 /  9.21 (9.00 / 9.21)   32768 x 3584  13.5 / 14.5 (13.6 / 14.5)
-//   17000 x 4096   9.02 /  9.84 (9.63 / 10.1)   32768 x 4096  14.7 / 15.8 (14.9 / 15.9)
-// and cached 22000 x 3072 10.1 / 10.5, 18500 x 3072 8.78 / 8.50.
+// pair-walking kernel, weights from HBM as a model's are (1.2 GB of copies):
+//   17000 x 2048   7.56 /  7.37    32768 x 2048  11.3 / 11.0
+//   16640 x 2816   8.37 /  8.29    40000 x 2816  14.9 / 14.6
+//   18500 x 3072   8.63 /  8.97    24576 x 3072  10.1 / 10.7
+//   18500 x 3584   9.27 /  9.70    32768 x 3584  13.5 / 14.5
+//   18500 x 4096   9.81 / 10.4     32768 x 4096  14.6 / 15.9
+//   18500 x 5632  13.2  / 14.1     32768 x 6144  20.8 / 22.3
+// A few such matrices alone stay in the last-level cache.  There the two are
+// level from 3584 to 4096 columns and at 6144 and the pair-walking kernel
+// takes 2 to 7 % less between (24576 x 4352 14.8 against 15.7) and below
+// (20000 x 3072 9.7 / 10.0, 17000 x 2048 7.2 / 8.1), so that rows of 3072 to
+// 3583 columns stream only where HBM decides more, past five chunks per wave.
 constexpr bool gemv_streams(int rows, int cols) {
     const int npos = stream_chunks_per_wave(rows);
     return cols <= 6144 && cols % 256 == 0 &&

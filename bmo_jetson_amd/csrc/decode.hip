@@ -12,17 +12,21 @@
 //
 // Work decomposition (gfx950, wave64).  S waves serve one (batch entry, query
 // head) unit and take contiguous pieces of its window; a workgroup holds one
-// unit, or R query heads of one kv head.  Batches with many units use one
-// wave per unit, smaller ones 2 to 8 so that enough waves run, merging in LDS
-// (a split across workgroups would have to merge through device-scope
-// atomics, which serialize across the XCDs).  The ring stores
-// slots in groups of G = 64 / LPK keys
+// unit, or R query heads of one kv head.  How many waves (1 to 8, merging in
+// LDS) and heads depends on the units, the window and whether the call
+// appends (decode_shape.hpp): many units or short windows mostly take one
+// wave, few units more, so that enough waves run (a split across workgroups
+// would have to merge through device-scope atomics, which serialize across
+// the XCDs).  The ring stores slots in groups of G = 64 / LPK keys
 // (ring_layout.hpp), LPK = head_dim / 32 blocks per key, so one group is one
 // wave iteration: lane l owns block l % LPK of key l / LPK and fetches its 16
 // K code bytes, 16 V code bytes and its (K, V) scale dword with three
 // coalesced loads from the group's 2304 contiguous bytes.  The loads are
-// nontemporal: every ring byte is read once per step and the working set is
-// far larger than the caches.  Each wave walks a contiguous run of groups,
+// nontemporal: a launch reads every ring byte once per workgroup that needs
+// it, and the working set is far larger than the caches.  (The R heads of a
+// workgroup walk the same groups in step, so all but the first find them in
+// the CU's cache in spite of it; with 4 heads a kv head in two workgroups of
+// 2 each byte comes from HBM twice.)  Each wave walks a contiguous run of groups,
 // keeping the loads of the next PF groups in flight while one group is
 // computed.  Keys past the window (and, fused, the slot being written) get
 // weight 0 by select.
@@ -355,8 +359,11 @@ __device__ __forceinline__ float half_of(uint32_t v) {
 // it as long as about kNewGroups groups: of two or four waves its run is
 // shorter by that many (taking the new token alone it would leave 1 of 2 and
 // 3 of 4 waves for the window: at 384 units of 32 groups, RoPE, 17.5 us a
-// launch with two waves and 10.8 with four, against 13.8 and 10.0); of eight
-// or more, whose runs are that short, it takes the new token alone.
+// launch with two waves and 10.8 with four, against 13.8 and 10.0).  Of eight
+// or more it takes the new token alone, on long windows too, where it could
+// share (3000 slots: 27 groups each of the other seven): these are the calls
+// of one session's layer loop, whose results the next layer quantizes again,
+// and their rounding stays as it is.
 constexpr int kNewGroups = 3;
 template <int NW, bool FUSED>
 __host__ __device__ constexpr int run_start(int w, int n_grp) {
@@ -635,16 +642,17 @@ __global__ __launch_bounds__(64 * R * S) void decode_kernel(DecodeParams p) {
     };
     // acc sums w * c with codes 0..15 and the -8 w of every key is owed until
     // the end (csum): over a long run that debt grows past the sums it is
-    // taken from, and their rounding with it.  It is paid, in 32 adds, after
-    // so many groups that a split's error against 64 bits is no larger than
-    // that of eight short runs: every 3 groups of two or four waves (32
+    // taken from, and their rounding with it.  It is paid, in 32 adds, every
+    // 3 groups of two or four waves (relative error against 64 bits, 32
     // groups, two waves: 4.9e-7 paid every 15, 4.4e-7 every 9, 3.8e-7 every
-    // 3; eight waves 4.0e-7; 25.6 us each; four waves: 4.3e-7 every 9, 3.7e-7
-    // every 3, 12 sessions 150.7 and 152.2 us), every 9 of grouped queries,
-    // which are bound by issue (32 heads of 8, 1024 slots: 111 us every 3,
-    // 107 every 9), every 6 of a long one-wave run, and once in a
-    // one-wave run of up to 40, where twice costs 0.3 % of the launch (32
-    // groups 6.3e-7 without, 5.3e-7 with).  Eight waves' runs are short.
+    // 3, 25.6 us each; four waves: 4.3e-7 every 9, 3.7e-7 every 3, 12
+    // sessions 150.7 and 152.2 us), every 9 of grouped queries, which are
+    // bound by issue (32 heads of 8, 1024 slots: 4.4e-7, 107 us; every 3 111
+    // us), every 6 of a long one-wave run (3000 slots 5.1e-7, 1.4e-6
+    // without), and once in a one-wave run of up to 40, where twice costs
+    // 0.3 % of the launch (32 groups 6.3e-7 without, 5.3e-7 with).  Eight
+    // waves do not pay before the end: 4.1e-7 at 512 slots and 5.9e-7 at
+    // 3000, where their runs are long (see run_start for why they stay).
     const int settle_every = S > 1 && R == 1 ? 1 : R > 1 ? 9 / NB : n_it <= 40 ? 24 / NB : 6 / NB;
     auto settle = [&]() {
         const float c = (-8.0f / 16777216.0f) * csum;

@@ -10,17 +10,20 @@
 // (src/bmo_compute.cpp:2188-2641) instead interleaves each layer's attention
 // with its own work on the handle's stream -- the QKV projection before it,
 // the output projection and FFN after it -- so the handle also takes one
-// layer at a time (begin_step, layer, end_step), asynchronously.  Either can
-// be captured into a HIP graph and replayed per token: capture_begin /
-// capture_end bracket whatever the caller enqueues on the handle's stream,
-// and the graph reads the position it begins at from device memory, so
-// replays keep attending (and rotating, with RoPE) at the current position.  A capture
-// may start with an asynchronous reset (the depformer's per-frame reset,
-// src/bmo_api.cpp:682) and hold several steps (its 8 codebook steps).  This
-// is what bmo_capture_graphs / bmo_has_cuda_graphs stand for
-// (src/bmo_api.cpp:334-359), whose static capture froze RoPE at the capture
-// position and was disabled; the reference keeps per-step depth graphs
-// (src/bmo_api.cpp:59-61,535-558).
+// layer at a time (begin_step, layer, end_step), asynchronously.
+//
+// Either can be kept and run again per token.  capture keeps a whole step's
+// buffers, and replay launches the step at the position it is given, which
+// the host knows.  capture_begin / capture_end record whatever the caller
+// enqueues on the handle's stream in between into a HIP graph, which reads
+// the position it begins at from device memory (after a recorded reset its
+// steps know theirs), so replays keep attending (and rotating, with RoPE) at
+// the current position.  A recording may hold an asynchronous reset (the
+// depformer's per-frame reset, src/bmo_api.cpp:682) and several steps (its 8
+// codebook steps).  This is what bmo_capture_graphs / bmo_has_cuda_graphs
+// stand for (src/bmo_api.cpp:334-359), whose static capture froze RoPE at the
+// capture position and was disabled; the reference keeps per-step depth
+// graphs (src/bmo_api.cpp:59-61,535-558).
 #include <hip/hip_runtime.h>
 
 #include <climits>

@@ -231,17 +231,18 @@ class KVRing:
 class Session:
     """Per-session handle (bmo_attn_session_*): one session of a ring with its
     own HIP stream and device position; ``forward`` runs one token's fused
-    append + attention through every layer at a position and advances it,
-    ``capture`` / ``replay`` do the same from a HIP graph recorded in the
-    library.  q/out are [n_layers][n_heads][head_dim] and k/v
+    append + attention through every layer at a position and advances it;
+    ``capture`` keeps a step's buffers and ``replay`` runs that step (every
+    layer in one launch, so all layers' q/k/v must be there when it begins).
+    q/out are [n_layers][n_heads][head_dim] and k/v
     [n_layers][n_kv_heads][head_dim] fp32 device buffers.
 
     At a model's layer granularity, ``begin_step(pos)``, ``layer(l, q, k, v,
     out)`` per layer and ``end_step()`` queue the step one layer at a time on
     ``stream``, where the caller's own kernels (projections, FFN) fall
     between them; ``capture_begin()`` / ``capture_end()`` record whatever is
-    queued on the stream in between (a frame may start with
-    ``reset_async()``), and ``replay`` runs it."""
+    queued on the stream in between into a HIP graph (a frame may start with
+    ``reset_async()``), and ``replay`` runs it instead."""
 
     def __init__(self, ring: KVRing, session: int, n_heads: int, scale: float = 0.0,
                  rope_theta: float = 0.0):

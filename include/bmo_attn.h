@@ -330,9 +330,12 @@ BMO_ATTN_API void *bmo_attn_session_stream(bmo_attn_session_t *s);
 /* One token step at position pos (0 <= pos <= 2^31 - 2; any position, not
  * only the next one, as bmo_forward_temporal2 takes it,
  * src/bmo_api.cpp:365-511), launched eagerly on the handle's stream, all
- * layers at once (one after another where out overlaps an input, so that a
- * layer then sees what the layers before it wrote); returns when out is
- * written.  Afterwards the position is pos + 1. */
+ * layers at once: every layer's q, k and v are there when it begins (a model
+ * whose layers feed one another uses the layer calls below).  Where out
+ * overlaps an input the layers run one after another, so that a layer then
+ * sees what the layers before it wrote.  The outputs are those of the layer
+ * calls bit for bit.  Returns when out is written; afterwards the position is
+ * pos + 1, or, after an error, what it was. */
 BMO_ATTN_API int bmo_attn_session_forward(bmo_attn_session_t *s, int pos, const float *q,
                                           const float *k, const float *v, float *out);
 
@@ -350,9 +353,8 @@ BMO_ATTN_API int bmo_attn_session_has_graph(bmo_attn_session_t *s);
 
 /* Runs the captured step (bmo_attn_session_capture) or replays the captured
  * graph (_capture_begin / _end) on the handle's stream and returns when it
- * is done; the captured
- * buffers hold the inputs on entry and the outputs on return.  A graph that
- * does not begin with a reset runs at position pos (same range as forward;
+ * is done; the captured buffers hold the inputs on entry and the outputs on
+ * return.  A graph that does not begin with a reset runs at position pos (same range as forward;
  * replaying at the handle's current position costs one graph launch, another
  * position first sets the device position) and leaves the position at pos +
  * its steps; a graph that begins with bmo_attn_session_reset_async ignores
@@ -436,8 +438,7 @@ BMO_ATTN_API const char *bmo_attn_session_last_error(bmo_attn_session_t *s);
  * aligned.  A 16-byte aligned W_dev with cols a multiple of 256, at most 6144
  * (past 16384 rows at least 3584, past 20480 at least 3072), takes a faster
  * streaming kernel; the outputs are the same bit for bit either way.
- * Asynchronous on stream.  Returns
- * BMO_ATTN_OK or an error code; rejected arguments launch nothing and are
+ * Asynchronous on stream.  Returns BMO_ATTN_OK or an error code; rejected arguments launch nothing and are
  * reported once on stderr (the reference's launcher returns nothing). */
 BMO_ATTN_API int bmo_launch_gemv_q4_0_q8_1(const void *W_dev, const float *x_dev,
                                            float *y_dev, int rows, int cols,

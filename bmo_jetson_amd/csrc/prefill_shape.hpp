@@ -26,8 +26,8 @@ constexpr StagedShape kStagedShapes[] = {{16, 1}, {16, 2}, {8, 1}, {8, 2}};
 // stand for other rings and for head_dim 64 too, though the window does not
 // enter: of 576 calls of 1 to 24 sessions (8 of 32 heads' K/V), 16 to 400
 // tokens, 512 slots empty and full and 2048 full, both head dims, none takes
-// longer than with 16 x 1 throughout but 12 sessions x 256 tokens on an empty
-// ring at d64 (31.1 against 30.0 us; full 52 / 57).
+// longer than in the build that had 16 x 1 alone but 12 sessions x 256 tokens
+// on an empty ring at d64 (31.1 against 30.0 us; full 52 / 57).
 constexpr double staged_cost(const StagedShape &s, int64_t workgroups) {
     const int per_cu = s.qw == 16 ? 1 : 2;
     const double alone = s.qw == 16 ? (s.ks == 1 ? 1.0 : 0.81) : (s.ks == 1 ? 0.88 : 0.71);

@@ -1,7 +1,8 @@
 """Waves per unit and groups in flight of the decode kernel against the float64
 oracle (|gpu - ref| <= 2e-3 + 1e-3 |ref|): the default rule near both sides of
-each of its lines (tests/test_decode_shapes.py has the lines themselves), and the shapes that it chooses, forced, at runs of no, one
-and few groups per wave."""
+each of its lines (tests/test_decode_shapes.py has the lines themselves), and
+the shapes that it chooses, forced, at runs of no, one and few groups per
+wave."""
 import numpy as np
 import pytest
 

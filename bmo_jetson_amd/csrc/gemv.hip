@@ -335,7 +335,7 @@ __global__ __launch_bounds__(512) void gemv_stream_kernel(GemvParams p) {
     // that are read (rows are a multiple of 16 bytes), and a wave without
     // chunks reads the last chunk
     auto issue = [&](int k, u32x4_t (&w)[NPC]) {
-        const int64_t cbase = (int64_t) min(c0 + k * stride, n_chunks - 1) * chunk_bytes;
+        const int64_t cbase = min((int64_t) c0 + (int64_t) k * stride, (int64_t) n_chunks - 1) * chunk_bytes;
         const int64_t last = min(cbase + chunk_bytes, mat_bytes) - 16;
 #pragma unroll
         for (int j = 0; j < NPC; ++j)
@@ -398,10 +398,10 @@ __global__ __launch_bounds__(512) void gemv_stream_kernel(GemvParams p) {
         if (lane == 0) {
 #pragma unroll
             for (int k = 0; k < NPOS; ++k) {
-                const uint32_t row = (uint32_t) (c0 + (k0 + k) * stride) * R;
+                const int64_t row = ((int64_t) c0 + (int64_t) (k0 + k) * stride) * R;
 #pragma unroll
                 for (int r = 0; r < R; ++r)
-                    if (k0 + k < n_mine && row + r < (uint32_t) p.rows) p.y[row + r] = yv[k][r];
+                    if (k0 + k < n_mine && row + r < p.rows) p.y[row + r] = yv[k][r];
             }
         }
     }

@@ -467,8 +467,8 @@ constexpr int stream_chunks_per_wave(int rows) {
 //   18500 x 4096   9.81 / 10.4     32768 x 4096  14.6 / 15.9
 //   18500 x 5632  13.2  / 14.1     32768 x 6144  20.8 / 22.3
 // A few such matrices alone stay in the last-level cache.  There the two are
-// level from 3584 to 4096 columns and at 6144 and the pair-walking kernel
-// takes 2 to 7 % less between (24576 x 4352 14.8 against 15.7) and below
+// within 3 % from 3584 to 4096 columns and at 6144 and the pair-walking kernel
+// takes 1 to 8 % less between (24576 x 4352 14.4 against 15.5) and below
 // (20000 x 3072 9.7 / 10.0, 17000 x 2048 7.2 / 8.1), so that rows of 3072 to
 // 3583 columns stream only where HBM decides more, past five chunks per wave.
 constexpr bool gemv_streams(int rows, int cols) {
